@@ -150,7 +150,26 @@ struct ScanCtx {
   float na[DS];
   float h[DS];
   float bdt, dd;
+  float xmax;  // see scan_x_max
 };
+
+// The largest softplus argument x for which every decay exponent na_n dt,
+// dt = softplus(x), stays at or above -126 (exp2_neg_core's range), capped
+// at ORDINARY: dt <= x + log 2 for x >= 0 and <= log 2 below, so x up to
+// 126 / max|na| - 0.7 qualifies, and none does where even dt = 0.7 is too
+// much (or a coefficient is NaN).
+template <int DS>
+__device__ __forceinline__ float scan_x_max(const float (&na)[DS]) {
+  float lo = 0.0f;
+  bool nan = false;
+#pragma unroll
+  for (int n = 0; n < DS; ++n) {
+    lo = __builtin_fminf(lo, na[n]);
+    nan = nan || na[n] != na[n];
+  }
+  const float x = 126.0f / -lo - 0.7f;  // lo = 0: inf
+  return !nan && x >= 0.0f ? __builtin_fminf(x, ORDINARY) : -__builtin_huge_valf();
+}
 
 template <int DS, int RB>
 __device__ __forceinline__ void scan_load(ScanCtx<DS, RB>& sc, const LayerW& Lw, const float* ssm,
@@ -166,6 +185,7 @@ __device__ __forceinline__ void scan_load(ScanCtx<DS, RB>& sc, const LayerW& Lw,
   }
   sc.bdt = Lw.b_dt[c];
   sc.dd = Lw.dd[c];
+  sc.xmax = scan_x_max<DS>(sc.na);
 }
 
 template <int DS, int RB>
@@ -200,43 +220,89 @@ template <int DS, int M>
 constexpr bool scan_fused_update() {
   return M == MATH_HW && (DS == 16 || BOA_SCAN_B16_FUSED_DS32);
 }
-// The channel's parameters come from P: wdt(j), na(n), bdt(), dd() (the
-// registers of a ScanCtx, or shared memory); h is updated in place.
-template <int DS, int RB, int M, class P>
-__device__ __forceinline__ float scan_token_p(float (&h)[DS], const P& p, const float* dt_in,
-                                              const float* bc, int r, float u, float z) {
-  float acc = 0.0f;
-#pragma unroll
-  for (int j = 0; j < RB; ++j)
-    if (j < r) acc = __builtin_fmaf(dt_in[j], p.wdt(j), acc);
-  const float dt = softplus<M>(acc + p.bdt());
-  const float* Bv = bc;
-  const float* Cv = bc + DS;
+// A token's x_proj row comes from an accessor: dt(j), B(n), C(n).
+template <int DS>
+struct RowFloats {  // floats: dt inputs, then B, then C
+  const float* d;
+  const float* bc;
+  __device__ __forceinline__ float dt(int j) const { return d[j]; }
+  __device__ __forceinline__ float B(int n) const { return bc[n]; }
+  __device__ __forceinline__ float C(int n) const { return bc[DS + n]; }
+  __device__ __forceinline__ void between(int) const {}
+};
+// One token's pass over a channel's states; CORE: the decay exponents need
+// no clamp.
+template <int DS, int M, bool CORE, class P, class Row>
+__device__ __forceinline__ float scan_states(float (&h)[DS], const P& p, const Row& row, float dt,
+                                             float u) {
   float y = 0.0f;
   if constexpr (scan_fused_update<DS, M>()) {
     const float dtu = dt * u;
 #pragma unroll
     for (int n = 0; n < DS; ++n) {
+      row.between(n);
       const float dA = exp2_neg_sel<M>(p.na(n) * dt);
-      h[n] = __builtin_fmaf(dA, h[n], Bv[n] * dtu);
-      y = __builtin_fmaf(h[n], Cv[n], y);
+      h[n] = __builtin_fmaf(dA, h[n], row.B(n) * dtu);
+      y = __builtin_fmaf(h[n], row.C(n), y);
     }
   } else {
 #pragma unroll
     for (int n = 0; n < DS; ++n) {
-      const float dA = exp2_neg_sel<M>(p.na(n) * dt);
-      const float dB = dt * Bv[n];
+      row.between(n);
+      const float e = p.na(n) * dt;
+      const float dA = M != MATH_HW && CORE ? exp2_neg_core(e) : exp2_neg_sel<M>(e);
+      const float dB = dt * row.B(n);
       h[n] = dA * h[n] + dB * u;
-      y = y + h[n] * Cv[n];
+      y = y + h[n] * row.C(n);
     }
   }
-  y = y + p.dd() * u;
-  float sg = rcp_sel<M>(1.0f + exp_sel<M>(-z));
-  return y * (z * sg);
+  return y;
+}
+// The channel's parameters come from P: wdt(j), na(n), bdt(), dd(), xmax()
+// (the registers of a ScanCtx, or shared memory); h is updated in place.
+template <int RB, class P, class Row>
+__device__ __forceinline__ float scan_x(const P& p, const Row& row, int r) {
+  float acc = 0.0f;
+#pragma unroll
+  for (int j = 0; j < RB; ++j)
+    if (j < r) acc = __builtin_fmaf(row.dt(j), p.wdt(j), acc);
+  return acc + p.bdt();
+}
+// whether a token runs without clamps and selects in the whole wave: every
+// lane's softplus and gate arguments ordinary, its decay exponents in range
+template <class P>
+__device__ __forceinline__ bool scan_ordinary(const P& p, float x, float z) {
+  return wave_ordinary((x >= -ORDINARY) & (x <= p.xmax()) & (__builtin_fabsf(z) <= ORDINARY));
+}
+// fp32, scan_ordinary tokens; CORE: p.xmax() bounds the decay exponents
+template <int DS, int M, bool CORE, class P, class Row>
+__device__ __forceinline__ float scan_token_ordinary(float (&h)[DS], const P& p, const Row& row,
+                                                     float x, float u, float z) {
+  const float y = scan_states<DS, M, CORE>(h, p, row, softplus_core(x), u) + p.dd() * u;
+  return y * (z * sigmoid_core(z));
+}
+// any token: the same values
+template <int DS, int M, class P, class Row>
+__device__ __forceinline__ float scan_token_any(float (&h)[DS], const P& p, const Row& row,
+                                                float x, float u, float z) {
+  const float dt = M == MATH_HW ? softplus<M>(x) : softplus_any<M>(x);
+  const float y = scan_states<DS, M, false>(h, p, row, dt, u) + p.dd() * u;
+  return y * (z * (M == MATH_HW ? sigmoid<M>(z) : sigmoid_any<M>(z)));
+}
+template <int DS, int RB, int M, class P>
+__device__ __forceinline__ float scan_token_p(float (&h)[DS], const P& p, const float* dt_in,
+                                              const float* bc, int r, float u, float z) {
+  const RowFloats<DS> row{dt_in, bc};
+  const float x = scan_x<RB>(p, row, r);
+  if (M != MATH_HW && scan_ordinary(p, x, z))
+    return scan_token_ordinary<DS, M, P::CORE>(h, p, row, x, u, z);
+  return scan_token_any<DS, M>(h, p, row, x, u, z);
 }
 template <int DS, int RB>
 struct ScanRegs {
   const ScanCtx<DS, RB>& c;
+  static constexpr bool CORE = true;
+  __device__ __forceinline__ float xmax() const { return c.xmax; }
   __device__ __forceinline__ float wdt(int j) const { return c.wdt[j]; }
   __device__ __forceinline__ float na(int n) const { return c.na[n]; }
   __device__ __forceinline__ float bdt() const { return c.bdt; }
@@ -252,6 +318,8 @@ template <int DS, int RB>
 struct ScanLds {
   const float* p;
   int cl;
+  static constexpr bool CORE = false;  // no per-channel limit kept: exp2_neg clamps
+  __device__ __forceinline__ float xmax() const { return ORDINARY; }
   __device__ __forceinline__ float na(int n) const { return p[((n >> 2) * 16 + cl) * 4 + (n & 3)]; }
   __device__ __forceinline__ float wdt(int j) const {
     return p[DS * 16 + ((j >> 2) * 16 + cl) * 4 + (j & 3)];

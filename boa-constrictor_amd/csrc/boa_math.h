@@ -38,21 +38,56 @@ BOA_DEV float ldv(const uint16_t* p) { return bf16_to_f32(*p); }
 BOA_DEV void stv(float* p, float v) { *p = v; }
 BOA_DEV void stv(uint16_t* p, float v) { *p = f32_to_bf16(v); }
 
-// e^x and log(y) in two forms with identical results for every input:
-// expf_ / logf_ are branch-free (the arithmetic runs on a clamped or rescaled
-// argument and selects give the special values, so a wavefront never
-// diverges), expf_br / logf_br return early on special values.  2^k is
-// applied with ldexp, which is exact here as the product with 2^k is (for
-// k = 128 either form overflows alike).  Long per-element chains (the chunk
-// scan) run faster branch-free; latency-bound kernels (the decode step) run
-// faster with the early returns.
+// What an fp32 element costs on gfx950 (a wave64 instruction's issue on one
+// SIMD, measured with independent chains): add, mul and fma on VGPRs,
+// literals or inline constants, integer add and the bit operations about 2.4
+// cycles; anything with an SGPR operand, min / max / med3, rounding,
+// conversions, shifts, ldexp, compares, selects and the div_ helpers 4.2; the
+// transcendentals 8.2.  fp32 MFMAs issue no faster than that and not beside
+// it (eight fma and one 16x16x4 MFMA take 22 + 34 cycles), so the functions
+// below prefer adds and fmas to the instructions named for a job:
+//   - rint(y), |y| < 2^22, is (y + 1.5 2^23) - 1.5 2^23, and the sum's low
+//     bits are the integer itself: p 2^k is an exponent-field add
+//     (v_lshl_add) instead of rndne + cvt + ldexp;
+//   - a division whose operands and quotient stay in the normal range needs
+//     no scaling and no fix-up (div_normal);
+//   - one comparison of the whole wave picks the form for ordinary arguments
+//     (no clamps, no selects) or the general one (wave_ordinary).
+// The results are those of the general forms for every float.
 
-// e^x for finite x in [-87, 88.7228...]
+// RINT_MAGIC + y: rint(y) in the low mantissa bits for |y| < 2^22.
+constexpr float RINT_MAGIC = 12582912.0f;
+// p 2^k for k = rint_sum - RINT_MAGIC; p, p 2^k normal (or p 2^k = 2^128 = inf).
+BOA_DEV float scale_rint(float p, float rint_sum) { return u2f(f2u(p) + (f2u(rint_sum) << 23)); }
+
+// n / d, correctly rounded, for normal d with a normal reciprocal and n / d
+// zero or normal by a margin of 2^24: Newton's step on the reciprocal, then
+// two residual corrections of the quotient (Markstein).  8 instructions, 27
+// cycles, against 12 and about 45 for the scaled division.
+BOA_DEV float div_normal(float n, float d) {
+  float y = __builtin_amdgcn_rcpf(d);
+  y = __builtin_fmaf(__builtin_fmaf(-d, y, 1.0f), y, y);
+  float q = n * y;
+  q = __builtin_fmaf(__builtin_fmaf(-d, q, n), y, q);
+  return __builtin_fmaf(__builtin_fmaf(-d, q, n), y, q);
+}
+
+// whether every active lane's predicate holds (a scalar branch, no divergence)
+BOA_DEV bool wave_ordinary(bool p) {
+  return __builtin_expect(__builtin_amdgcn_ballot_w64(!p) == 0, 1);
+}
+
+// e^x and log(y): expf_ is branch-free (the arithmetic runs on a clamped
+// argument and selects give the special values), expf_br returns early on
+// them; the results are the same for every input.
+
+// e^x for x in [-87, 88.7228...), where it is finite
 BOA_DEV float exp_core(float x) {
   const float LOG2E = 1.44269504088896340736f;
   const float LN2_HI = 0.693147182464599609375f;
   const float LN2_LO = -1.904654323148236e-09f;
-  const float kf = __builtin_rintf(x * LOG2E);
+  const float km = x * LOG2E + RINT_MAGIC;
+  const float kf = km - RINT_MAGIC;
   float r = __builtin_fmaf(-kf, LN2_HI, x);
   r = __builtin_fmaf(-kf, LN2_LO, r);
   float p = 1.98412698412698412698e-4f;
@@ -63,13 +98,13 @@ BOA_DEV float exp_core(float x) {
   p = __builtin_fmaf(p, r, 0.5f);
   p = __builtin_fmaf(p, r, 1.0f);
   p = __builtin_fmaf(p, r, 1.0f);
-  return __builtin_ldexpf(p, (int)kf);
+  return scale_rint(p, km);
 }
 
 BOA_DEV float expf_(float x) {
   float res = exp_core(__builtin_fminf(__builtin_fmaxf(x, -87.0f), 88.72283935546875f));
   res = x < -87.0f ? 0.0f : res;
-  res = x > 88.72283935546875f ? __builtin_huge_valf() : res;
+  res = x >= 88.72283935546875f ? __builtin_huge_valf() : res;
   return x != x ? x : res;
 }
 
@@ -81,12 +116,13 @@ BOA_DEV float expf_(float x) {
 // [-126, 0] (fmaxf turns a NaN into -126), split as k + r with k = rint(t)
 // and r = t - k in [-1/2, 1/2] (exact); 2^r comes from a degree-6
 // polynomial with 2^0 = 1 exact, fitted to the relative error of 2^r on
-// [-1/2, 1/2] (under one ulp with fp32 fma evaluation), and 2^k is applied
-// with ldexp.  The least result is 2^-126: no subnormal is produced.
-BOA_DEV float exp2_neg(float t) {
-  const float s = __builtin_fminf(__builtin_fmaxf(t, -126.0f), 0.0f);
-  const float k = __builtin_rintf(s);
-  const float r = s - k;
+// [-1/2, 1/2] (under one ulp with fp32 fma evaluation), and 2^k is added to
+// the exponent field.  The least result is 2^-126: no subnormal is produced.
+// exp2_neg_core: t already in [-126, 0] (29 cycles an element, against 37
+// with the clamp, rndne, cvt and ldexp).
+BOA_DEV float exp2_neg_core(float s) {
+  const float km = s + RINT_MAGIC;
+  const float r = s - (km - RINT_MAGIC);
   float p = 0x1.41fbbap-13f;
   p = __builtin_fmaf(p, r, 0x1.5f3e54p-10f);
   p = __builtin_fmaf(p, r, 0x1.3b2d4cp-7f);
@@ -94,53 +130,37 @@ BOA_DEV float exp2_neg(float t) {
   p = __builtin_fmaf(p, r, 0x1.ebfbdcp-3f);
   p = __builtin_fmaf(p, r, 0x1.62e430p-1f);
   p = __builtin_fmaf(p, r, 1.0f);
-  return __builtin_ldexpf(p, (int)k);
+  return scale_rint(p, km);
+}
+BOA_DEV float exp2_neg(float t) {
+  return exp2_neg_core(__builtin_fminf(__builtin_fmaxf(t, -126.0f), 0.0f));
 }
 
 BOA_DEV float expf_br(float x) {
   if (x != x) return x;
-  if (x > 88.72283935546875f) return __builtin_huge_valf();
+  if (x >= 88.72283935546875f) return __builtin_huge_valf();
   if (x < -87.0f) return 0.0f;
   return exp_core(x);
 }
 
-// log(y) for y > 0 finite (subnormals rescaled)
+// log(y) for y in [1, 2^127): y = 2^e m with m in (sqrt(1/2), sqrt(2)]
 BOA_DEV float log_core(float y) {
-  const bool sub = (f2u(y) >> 23) == 0;
-  const uint32_t u = f2u(sub ? y * 8388608.0f : y);
-  int e = (int)(u >> 23) - 127 - (sub ? 23 : 0);
-  float m = u2f((u & 0x007FFFFFu) | 0x3F800000u);
-  const bool hi = m > 1.41421353816986083984375f;
-  m = hi ? m * 0.5f : m;
-  e = hi ? e + 1 : e;
-  float s = (m - 1.0f) / (m + 1.0f);
-  float s2 = s * s;
+  const uint32_t above = f2u(y) - 0x3F3504F4u;  // from the least float over sqrt(1/2)
+  const int e = (int)above >> 23;
+  const float m = u2f(f2u(y) - (above & 0xFF800000u));
+  const float s = div_normal(m - 1.0f, m + 1.0f);
+  const float s2 = s * s;
   float p = 0.0909090909090909090909f;
   p = __builtin_fmaf(p, s2, 0.111111111111111111111f);
   p = __builtin_fmaf(p, s2, 0.142857142857142857143f);
   p = __builtin_fmaf(p, s2, 0.2f);
   p = __builtin_fmaf(p, s2, 0.333333333333333333333f);
-  float two_s = s + s;
-  float lm = __builtin_fmaf(two_s * s2, p, two_s);
+  const float two_s = s + s;
+  const float lm = __builtin_fmaf(two_s * s2, p, two_s);
   const float LN2_HI = 0.693147182464599609375f;
   const float LN2_LO = -1.904654323148236e-09f;
-  float ef = (float)e;
+  const float ef = (float)e;
   return __builtin_fmaf(ef, LN2_HI, __builtin_fmaf(ef, LN2_LO, lm));
-}
-
-BOA_DEV float logf_(float y) {
-  float res = log_core(y);
-  res = y == 0.0f ? -__builtin_huge_valf() : res;
-  res = y < 0.0f ? __builtin_nanf("") : res;
-  res = y == __builtin_huge_valf() ? y : res;
-  return y != y ? y : res;
-}
-
-BOA_DEV float logf_br(float y) {
-  if (y != y) return y;
-  if (y == __builtin_huge_valf()) return y;
-  if (y <= 0.0f) return (y == 0.0f) ? -__builtin_huge_valf() : __builtin_nanf("");
-  return log_core(y);
 }
 
 // Forms of the transcendental activations.  MATH_BF and MATH_BR give
@@ -158,15 +178,29 @@ BOA_DEV float hw_rcp(float x) { return __builtin_amdgcn_rcpf(x); }
 
 template <int M>
 BOA_DEV float exp_sel(float x) { return M == MATH_HW ? hw_exp(x) : M == MATH_BR ? expf_br(x) : expf_(x); }
-template <int M>
-BOA_DEV float log_sel(float x) { return M == MATH_HW ? hw_log(x) : M == MATH_BR ? logf_br(x) : logf_(x); }
-template <int M>
-BOA_DEV float rcp_sel(float x) { return M == MATH_HW ? hw_rcp(x) : 1.0f / x; }
 
-// activations.hpp:33-84 (device branch); core for x in [-88, 88]
+// |x| up to which sigmoid_core and softplus_core hold: e^87 < 2^126, so
+// 1 + e^x and its reciprocal are normal
+constexpr float ORDINARY = 87.0f;
+// 1 / (1 + e^-x) and log(1 + e^x) for |x| <= ORDINARY
+BOA_DEV float sigmoid_core(float x) { return div_normal(1.0f, 1.0f + exp_core(-x)); }
+BOA_DEV float softplus_core(float x) { return log_core(1.0f + exp_core(x)); }
+// ... and for every x: e^x = 0 below -87 leaves 1 + 0, whose log is 0; above
+// 88.72 it is inf, whose log is inf and reciprocal 0
+template <int M>
+BOA_DEV float sigmoid_any(float x) { return 1.0f / (1.0f + exp_sel<M>(-x)); }
+template <int M>
+BOA_DEV float softplus_any(float x) {
+  const float c = log_core(1.0f + exp_core(__builtin_fminf(__builtin_fmaxf(x, -87.0f), 87.0f)));
+  if (__builtin_fabsf(x) <= ORDINARY) return c;
+  const float y = 1.0f + exp_sel<M>(x);  // 1, [2^125, 2^128), inf or NaN
+  return y < __builtin_huge_valf() ? log_core(y) : y;
+}
+
+// activations.hpp:33-84 (device branch) for x in [-20, 20], the arguments
+// that tanh's saturation leaves
 BOA_DEV float repro_exp_core(float x) {
-  float kf = __builtin_floorf(x * 1.44269504088896340736f + 0.5f);
-  int k = (int)kf;
+  const float kf = __builtin_floorf(x * 1.44269504088896340736f + 0.5f);
   float r = x + (-(kf * 0.69314718055994530942f));
   float t = 0.008333333333f + r * 0.001388888889f;
   t = 0.041666666667f + r * t;
@@ -174,31 +208,24 @@ BOA_DEV float repro_exp_core(float x) {
   t = 0.5f + r * t;
   t = 1.0f + r * t;
   t = 1.0f + r * t;
-  return t * u2f((uint32_t)((k + 127) << 23));
+  return scale_rint(t, kf + RINT_MAGIC);
 }
 
-template <int M>
-BOA_DEV float repro_exp(float x) {
-  if (M == MATH_HW) return hw_exp(x);
-  if (M == MATH_BR) {
-    if (x <= -88.0f) return 0.0f;
-    return repro_exp_core(x >= 88.0f ? 88.0f : x);
-  }
-  const float res = repro_exp_core(__builtin_fminf(__builtin_fmaxf(x, -88.0f), 88.0f));
-  return x <= -88.0f ? 0.0f : (x != x ? x : res);
-}
-
-// activations.hpp:87-98
+// activations.hpp:87-98: (e^2x - 1) / (e^2x + 1), and +-1 where |x| > 10.
+// The quotient at +-10 is +-1 exactly (e^20 +- 1 and e^-20 +- 1 round to
+// e^20 and to +-1), so clamping x to [-10, 10] gives the saturation without
+// selects; a NaN is left to the caller's product with x.  In hardware
+// arithmetic 1 - 2 / (e^2x + 1) saturates by itself.
 template <int M>
 BOA_DEV float repro_tanh(float x) {
-  const float ax = x < 0.0f ? -x : x;
-  if (M == MATH_BR && ax > 10.0f) return (x > 0.0f) ? 1.0f : -1.0f;
-  const float e2x = repro_exp<M>(2.0f * x);
-  const float th = M == MATH_HW ? 1.0f - 2.0f * hw_rcp(e2x + 1.0f) : (e2x + -1.0f) / (e2x + 1.0f);
-  return ax > 10.0f ? ((x > 0.0f) ? 1.0f : -1.0f) : th;
+  if (M == MATH_HW) return __builtin_fmaf(-2.0f, hw_rcp(hw_exp(2.0f * x) + 1.0f), 1.0f);
+  const float e2x = repro_exp_core(2.0f * __builtin_fminf(__builtin_fmaxf(x, -10.0f), 10.0f));
+  return div_normal(e2x + -1.0f, e2x + 1.0f);
 }
 
-// activations.hpp:105-117 (tanh GELU used by the FF epilogue)
+// activations.hpp:105-117 (tanh GELU used by the FF epilogue).  fp32 on
+// gfx950: about 106 cycles an element against 160 with the selects and the
+// scaled division.
 template <int M = MATH_BF>
 BOA_DEV float gelu(float x) {
   float cube = (x * x) * x;
@@ -207,16 +234,23 @@ BOA_DEV float gelu(float x) {
   return 0.5f * (x * (1.0f + th));
 }
 
+// 1 / (1 + exp(-x)) of the gate and SiLU
+template <int M = MATH_BF>
+BOA_DEV float sigmoid(float x) {
+  if (M == MATH_HW) return hw_rcp(1.0f + hw_exp(-x));
+  return wave_ordinary(__builtin_fabsf(x) <= ORDINARY) ? sigmoid_core(x) : sigmoid_any<M>(x);
+}
+
 // SiLU in the form v * (1 / (1 + exp(-v))) (mamba_kernels.cu:188-189)
 template <int M = MATH_BF>
-BOA_DEV float silu(float x) {
-  float sg = rcp_sel<M>(1.0f + exp_sel<M>(-x));
-  return x * sg;
-}
+BOA_DEV float silu(float x) { return x * sigmoid<M>(x); }
 
 // unthresholded softplus log(1 + exp(x)) (inference_kernels.cu:376-382)
 template <int M = MATH_BF>
-BOA_DEV float softplus(float x) { return log_sel<M>(1.0f + exp_sel<M>(x)); }
+BOA_DEV float softplus(float x) {
+  if (M == MATH_HW) return hw_log(1.0f + hw_exp(x));
+  return wave_ordinary(__builtin_fabsf(x) <= ORDINARY) ? softplus_core(x) : softplus_any<M>(x);
+}
 
 // 2^t for t <= 0 (see exp2_neg) in the chosen form
 template <int M>

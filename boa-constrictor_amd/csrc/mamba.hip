@@ -553,68 +553,164 @@ hipError_t launch_conv_chunk(const void* xz, float* conv_state, const float* w, 
 }
 
 // -------------------------------------------------------- selective scan
-// Thread per (lane, channel); a block covers bs channels of one lane (bs
-// divides di), so the token's delta row (dt_in | B | C) is the same for every
-// thread of the wave and is read with scalar loads into SGPRs: no LDS
-// staging and no barriers (against rows staged in LDS and read as
-// broadcasts, 9 % faster in fp32 on the C2 model and 19-21 % in bf16 on the
-// C3 and C5 models).  FULL: dt_rank equals the bound RB.  Otherwise the dt
-// inputs beyond dt_rank are zeroed, which leaves the fma chain's value
-// unchanged (the partial sum starts at +0 and so is never -0, and
-// fma(0, 0, a) = a).  d_state 16 with dt_rank <= 16 runs five (fp32, 80
-// VGPRs) or six (bf16) waves per SIMD.
+// Thread per (lane, channel); a block covers bs channels of one lane, so the
+// token's delta row (dt_in | B | C) is the same for every thread of the wave
+// and is read with scalar loads into SGPRs: no LDS staging and no barriers
+// (against rows staged in LDS and read as broadcasts, 9 % faster in fp32 on
+// the C2 model and 19-21 % in bf16 on the C3 and C5 models).  FULL: dt_rank
+// equals the bound RB.  Otherwise the dt inputs beyond dt_rank are zeroed,
+// which leaves the fma chain's value unchanged (the partial sum starts at +0
+// and so is never -0, and fma(0, 0, a) = a).
+// Bound by VALU issue (costs per instruction in boa_math.h).  A token of 64
+// channels by that count, and measured per compress pass: C2 (1000 lanes x
+// 2085 B) 1312 -> 1015 cycles, 71.1 -> 62.9 ms (fast forms for ordinary
+// tokens, no vector address arithmetic); C3 (8192 x 512 B) 555 -> 483, 57.1
+// -> 52.6 ms; C5 (4096 x 256 B) 1218 -> 1127, 102.7 -> 94.4 ms (no SGPRs
+// spilled to VGPR lanes).  Waves per SIMD: fp32 eight (64 VGPRs; seven
+// measured 64.1 ms, C2's 8000 waves then leaving an almost empty second
+// round), bf16 seven at d_state 16 (74 VGPRs and six waves 55.1 ms, eight
+// spill: 91.5) and four at d_state 32 (five spill: 128).
+template <int DS, int RB, bool FULL, typename TA>
+struct ScanRow;
 template <int DS, int RB, bool FULL>
-__device__ __forceinline__ void scan_row(const float* dr, int r, float* dv) {
+struct ScanRow<DS, RB, FULL, float> {
+  float d[RB], bc[2 * DS];
+  __device__ __forceinline__ ScanRow(__attribute__((address_space(4))) const float* dr, int r) {
 #pragma unroll
-  for (int j = 0; j < RB; ++j) {
-    const float v = dr[j];  // j < RB <= R: inside the row
-    dv[j] = FULL || j < r ? v : 0.0f;
+    for (int j = 0; j < RB; ++j) {
+      const float v = dr[j];  // j < RB <= R: inside the row
+      d[j] = FULL || j < r ? v : 0.0f;
+    }
+#pragma unroll
+    for (int j = 0; j < 2 * DS; ++j) bc[j] = dr[r + j];
   }
-#pragma unroll
-  for (int j = 0; j < 2 * DS; ++j) dv[RB + j] = dr[r + j];
-}
+  __device__ __forceinline__ float dt(int j) const { return d[j]; }
+  __device__ __forceinline__ float B(int n) const { return bc[n]; }
+  __device__ __forceinline__ float C(int n) const { return bc[DS + n]; }
+  __device__ __forceinline__ void between(int) const {}
+};
 // bf16 rows: dt_rank, d_state and so the row length are even (d_model is a
-// multiple of 64), so the element pairs are read as aligned dwords
+// multiple of 64), so the element pairs are read as aligned dwords, widened
+// by scalar instructions where an element is used.  At d_state 32 a row's 96
+// floats would not fit the SGPRs (the compiler spilled them to VGPR lanes,
+// 14 v_readlane a token): there the widening stays within groups of eight
+// states.
 template <int DS, int RB, bool FULL>
-__device__ __forceinline__ void scan_row(const uint16_t* dr, int r, float* dv) {
-  const uint32_t* w = reinterpret_cast<const uint32_t*>(dr);
+struct ScanRow<DS, RB, FULL, uint16_t> {
+  uint32_t w[RB / 2], wbc[DS];
+  int r;
+  __device__ __forceinline__ ScanRow(__attribute__((address_space(4))) const uint16_t* dr, int r_)
+      : r(r_) {
+    typedef __attribute__((address_space(4))) const uint32_t* Words;
 #pragma unroll
-  for (int j = 0; j < RB / 2; ++j) {
-    const uint32_t v = w[j];
-    dv[2 * j] = FULL || 2 * j < r ? u2f(v << 16) : 0.0f;
-    dv[2 * j + 1] = FULL || 2 * j + 1 < r ? u2f(v & 0xFFFF0000u) : 0.0f;
-  }
-  const uint32_t* wb = reinterpret_cast<const uint32_t*>(dr + r);
+    for (int j = 0; j < RB / 2; ++j) w[j] = ((Words)dr)[j];
 #pragma unroll
-  for (int j = 0; j < DS; ++j) {
-    const uint32_t v = wb[j];
-    dv[RB + 2 * j] = u2f(v << 16);
-    dv[RB + 2 * j + 1] = u2f(v & 0xFFFF0000u);
+    for (int j = 0; j < DS; ++j) wbc[j] = ((Words)(dr + r))[j];
   }
-}
+  static __device__ __forceinline__ float half_of(uint32_t v, int odd) {
+    return u2f(odd ? v & 0xFFFF0000u : v << 16);
+  }
+  __device__ __forceinline__ float dt(int j) const {
+    return FULL || j < r ? half_of(w[j / 2], j & 1) : 0.0f;
+  }
+  __device__ __forceinline__ float B(int n) const { return half_of(wbc[n / 2], n & 1); }
+  __device__ __forceinline__ float C(int n) const { return half_of(wbc[(DS + n) / 2], n & 1); }
+  __device__ __forceinline__ void between(int n) const {
+    if (n % 8 == 0) __builtin_amdgcn_sched_barrier(0);
+  }
+};
+
+// One lane's rows of an activation array behind a buffer descriptor.
+template <typename TA>
+struct RowBuf {
+  __amdgpu_buffer_rsrc_t rsrc;
+  __device__ __forceinline__ explicit RowBuf(const TA* base)
+      : rsrc(__builtin_amdgcn_make_buffer_rsrc(const_cast<TA*>(base), (short)0, -1, 0x00027000)) {}
+  __device__ __forceinline__ float load(int off, int row) const {
+    if constexpr (sizeof(TA) == 4)
+      return u2f(__builtin_amdgcn_raw_buffer_load_b32(rsrc, off, row, 0));
+    else
+      return bf16_to_f32(__builtin_amdgcn_raw_buffer_load_b16(rsrc, off, row, 0));
+  }
+  __device__ __forceinline__ void store(int off, int row, float v) const {
+    if constexpr (sizeof(TA) == 4)
+      __builtin_amdgcn_raw_buffer_store_b32(f2u(v), rsrc, off, row, 0);
+    else
+      __builtin_amdgcn_raw_buffer_store_b16(f32_to_bf16(v), rsrc, off, row, 0);
+  }
+};
 
 template <int DS, int RB, bool FULL, typename TA>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(DS == 16 && RB <= 16 ? (sizeof(TA) == 2 ? 6 : 5) : 1, 8)))
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(DS == 16 && RB <= 16 ? (sizeof(TA) == 2 ? 7 : 8) : (sizeof(TA) == 2 ? 4 : 1), 8)))
 void scan_chunk_sload_kernel(Dims D, LayerW Lw, const TA* __restrict__ xz,
                              const TA* __restrict__ conv, const TA* __restrict__ delta,
                              float* __restrict__ ssm_state, TA* __restrict__ y, int lanes,
                              int T) {
   const int di = D.di, R = D.R;
-  const int base = blockIdx.x * blockDim.x;
-  const int b = base / di;
-  const int c = base - b * di + threadIdx.x;
-  float* ssm = ssm_state + (size_t)(base + threadIdx.x) * DS;
+  const int per = (di + blockDim.x - 1) / blockDim.x;  // blocks per lane
+  const int b = blockIdx.x / per;
+  const unsigned c = (blockIdx.x - b * per) * blockDim.x + threadIdx.x;
+  if (c >= (unsigned)di) return;  // no barriers below
+  float* ssm = ssm_state + ((size_t)b * di + c) * DS;
+  constexpr int M = sizeof(TA) == 2 ? MATH_HW : MATH_BF;
   ScanCtx<DS, RB> sc;
   scan_load<DS, RB>(sc, Lw, ssm, c, di, D.r);
-  const TA* drows = delta + (size_t)b * T * R;
-  for (int t = 0; t < T; ++t) {
-    const size_t row = (size_t)b * T + t;
-    float dv[RB + 2 * DS];
-    scan_row<DS, RB, FULL>(drows + (size_t)t * R, D.r, dv);
-    const float u = ldv(conv + row * di + c);
-    const float z = ldv(xz + row * 2 * di + di + c);
-    stv(y + row * di + c, scan_token<DS, RB, sizeof(TA) == 2 ? MATH_HW : MATH_BF>(
-                              sc, dv, dv + RB, RB, u, z));
+  // the delta rows are read-only here: constant address space, scalar loads
+  typedef __attribute__((address_space(4))) const TA* CIn;
+  CIn drows = (CIn)(delta + (size_t)b * T * R);
+  // u, z and y through buffer accesses: a lane's byte offset in the row is
+  // constant and the row's offset a scalar, so a token costs no vector
+  // address arithmetic.  A lane's rows span under 2^32 bytes: with 65,536
+  // channels in flight (the dispatch's lower bound) their activations would
+  // otherwise exceed the card's memory 100 times.
+  const RowBuf<TA> ub(conv + (size_t)b * T * di), zb(xz + ((size_t)b * T * 2 + 1) * di),
+      yb(y + (size_t)b * T * di);
+  const int off = (int)(c * sizeof(TA)), row = di * (int)sizeof(TA);
+  int at = 0;  // the token's row in conv and y; twice that in xz
+  const ScanRegs<DS, RB> p{sc};
+  auto advance = [&] {
+    drows += R;
+    at = (int)((unsigned)at + (unsigned)row);
+  };
+  if constexpr (M == MATH_HW) {
+    auto token = [&] {
+      const ScanRow<DS, RB, FULL, TA> dv(drows, D.r);
+      const float u = ub.load(off, at), z = zb.load(off, (int)(2u * (unsigned)at));
+      yb.store(off, at, scan_token_any<DS, M>(sc.h, p, dv, scan_x<RB>(p, dv, RB), u, z));
+      advance();
+    };
+    int t = 0;
+    // two tokens an iteration where the update is fused: its fmas write
+    // another register than the state they read, and one token an iteration
+    // pays a copy per state
+    if constexpr (scan_fused_update<DS, M>())
+      for (; t + 2 <= T; t += 2) {
+        token();
+        token();
+      }
+    for (; t < T; ++t) token();
+  } else {
+    // runs of ordinary tokens; a token that is not one goes through the
+    // general form between them (outside the loop, so that the state stays
+    // in its registers)
+    int t = 0;
+    while (t < T) {
+      for (; t < T; ++t) {
+        const ScanRow<DS, RB, FULL, TA> dv(drows, D.r);
+        const float u = ub.load(off, at), z = zb.load(off, (int)(2u * (unsigned)at));
+        const float x = scan_x<RB>(p, dv, RB);
+        if (!scan_ordinary(p, x, z)) break;
+        yb.store(off, at, scan_token_ordinary<DS, M, true>(sc.h, p, dv, x, u, z));
+        advance();
+      }
+      if (t < T) {
+        const ScanRow<DS, RB, FULL, TA> dv(drows, D.r);
+        const float u = ub.load(off, at), z = zb.load(off, (int)(2u * (unsigned)at));
+        yb.store(off, at, scan_token_any<DS, M>(sc.h, p, dv, scan_x<RB>(p, dv, RB), u, z));
+        advance();
+        ++t;
+      }
+    }
   }
   scan_store<DS, RB>(sc, ssm);
 }
@@ -744,7 +840,7 @@ __global__ __launch_bounds__(256) void scan_chunk_tblk_kernel(Dims D, LayerW Lw,
         for (int j = 0; j < RB; ++j)
           if (j < r) acc = __builtin_fmaf(dv[j], wdt[j], acc);
         const float dt = softplus<M>(acc + bdt);
-        const float sg = rcp_sel<M>(1.0f + exp_sel<M>(-cz[i]));
+        const float sg = sigmoid<M>(cz[i]);
         *reinterpret_cast<float4*>(s_tok + 4 * tok) =
             make_float4(dt, scan_fused_update<DS, M>() ? dt * cu[i] : cu[i], dd * cu[i], cz[i] * sg);
       }
@@ -789,11 +885,12 @@ __global__ __launch_bounds__(256) void scan_chunk_tblk_kernel(Dims D, LayerW Lw,
   for (int n = 0; n < SPT; ++n) ssm[n] = h[n];
 }
 
-static int block_for(int di) {
-  for (int bs = 256; bs >= 32; bs >>= 1)
-    if (di % bs == 0) return bs;
-  return 0;
-}
+// Threads per block of the large-grid scan: whole waves of one lane's
+// channels, at most four.  At 160 channels (d_model 80) that is 192, the
+// last wave half idle; blocks of 32 threads, which divide 160, ran five
+// half-idle waves a lane instead of three (512 lanes x 3001 B: scan 10.9 ->
+// 9.2 ms per compress).
+static int block_for(int di) { return std::min(256, (di + 63) / 64 * 64); }
 
 #ifndef BOA_SCAN_TBLK_BELOW
 #define BOA_SCAN_TBLK_BELOW (64 * 1024)  // threads: one wave per SIMD
@@ -803,7 +900,7 @@ template <int DS, int RB>
 static hipError_t scan_chunk_go(const Dims& D, const LayerW& Lw, const void* xz, const void* conv,
                                 const void* delta, float* ssm_state, void* y, int lanes, int T,
                                 int bs, bool bf16, hipStream_t s) {
-  const dim3 grid((lanes * D.di) / bs);
+  const dim3 grid(lanes * ((D.di + bs - 1) / bs));
   if ((int64_t)lanes * D.di < BOA_SCAN_TBLK_BELOW) {
     if (D.di % TBK_CPB) return hipErrorInvalidValue;
     const size_t lds = sizeof(float) * TblkShape<DS>::template lds_floats<RB>();
@@ -852,7 +949,7 @@ hipError_t launch_scan_chunk(const Dims& D, const LayerW& Lw, const void* xz, co
                              const void* delta, float* ssm_state, void* y, int lanes, int T,
                              bool bf16, hipStream_t s) {
   const int bs = block_for(D.di);
-  if (!bs || D.r > RMAX || (D.ds != 16 && D.ds != 32)) return hipErrorInvalidValue;
+  if (D.r > RMAX || (D.ds != 16 && D.ds != 32)) return hipErrorInvalidValue;
   BOA_SCAN_DISPATCH(scan_chunk_go, D, Lw, xz, conv, delta, ssm_state, y, lanes, T, bs, bf16, s);
 }
 
