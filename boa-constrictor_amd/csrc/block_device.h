@@ -105,6 +105,26 @@ __device__ __forceinline__ lds_u32x4 lds_read128(const void* p) {
   asm volatile("ds_read_b128 %0, %1" : "=v"(v) : "v"(a) : "memory");
   return v;
 }
+// ... at LDS byte address a + OFF (the instruction's own offset)
+template <int OFF>
+__device__ __forceinline__ lds_u32x4 lds_read128_at(uint32_t a) {
+  lds_u32x4 v;
+  asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(v) : "v"(a), "n"(OFF) : "memory");
+  return v;
+}
+template <int OFF>
+__device__ __forceinline__ void lds_write64_at(uint32_t a, uint32_t lo, uint32_t hi) {
+  typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+  const u32x2 v = {lo, hi};
+  asm volatile("ds_write_b64 %0, %1 offset:%2" ::"v"(a), "v"(v), "n"(OFF) : "memory");
+}
+template <int OFF>
+__device__ __forceinline__ void lds_write128_at(uint32_t a, lds_u32x4 v) {
+  asm volatile("ds_write_b128 %0, %1 offset:%2" ::"v"(a), "v"(v), "n"(OFF) : "memory");
+}
+__device__ __forceinline__ uint32_t lds_addr(const void* p) {
+  return (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) void*)p;
+}
 __device__ __forceinline__ void lds_barrier() { asm volatile("s_barrier" ::: "memory"); }
 // the reads' values are the asm's outputs, so nothing uses them before it
 __device__ __forceinline__ void lds_wait4(lds_u32x4& a, lds_u32x4& b, lds_u32x4& c, lds_u32x4& d) {

@@ -16,6 +16,10 @@
 // activations the B operand (16 m-columns); a lane's accumulators are 4
 // consecutive n of one row m.  LDS: [rows][BK + 8] u16 per operand (the pad
 // staggers 16-byte row reads across banks), double-buffered.
+#include <algorithm>
+#include <type_traits>
+
+#include "block_device.h"
 #include "boa_kernels.h"
 #include "coder_device.h"
 
@@ -251,17 +255,348 @@ static hipError_t launch_b16(const GemmB16Args& a, hipStream_t s, int swizzle = 
   return hipGetLastError();
 }
 
+// ------------------------------------------------------- persistent blocks
+// 256 rows x 256 features a tile, eight waves of 64 x 128 (128 accumulators,
+// two waves per SIMD), one block per CU that walks over tiles.  What the
+// shape is chosen for, on MI355X:
+//   - LDS: a k-step's 32 MFMAs of a wave read 12 fragments (1 KB each); the
+//     64 x 64 wave tiles of gemm_bf16_kernel read 8 for 16, which alone
+//     filled the LDS.
+//   - Vector memory: 64-k stages of 128-byte rows are copied straight to LDS
+//     (global rows as whole cache lines).  Fragments loaded to registers
+//     instead (64-byte pieces of 16 rows) kept the texture-address units 86 %
+//     busy at a third of the MFMA rate.
+//   - Stores: a lane holds four features of a row; stored from there a wave
+//     writes 32-byte pieces of 16 rows, and those took longer than a short K
+//     loop (262,144 x 1024, K = 256: 368 us, 175 without them).  The tile
+//     turns round in LDS, 16 rows x 128 bytes at a time per wave, and leaves
+//     in whole lines.
+//   - K is short (256 to 2048): the next tile's first stage is copied while
+//     this tile's last one is multiplied and its epilogue runs.
+// LDS: two 64 KB stages (activations, then weights; the 16-byte chunk c of
+// row r at slot c ^ (r & 7), so that eight lanes of a fragment read hit eight
+// slots), 2 KB per wave for the epilogue, the bias of every feature.
+// The chains are gemm_bf16_kernel's (k-steps of 32 in ascending order), and
+// so are the bits.
+constexpr int GP_STAGE = 65536, GP_EPI = 2048, GP_MAX_N = 2048;
+constexpr int GP_LDS = 2 * GP_STAGE + 8 * GP_EPI + 4 * GP_MAX_N + 256;
+
+struct GpTile {
+  __amdgpu_buffer_rsrc_t x, w;  // the tile's activation rows, the wave's weight rows
+  int m, n;
+};
+
+template <int ACT, bool F32>
+__global__ __launch_bounds__(512, 2) void gemm_bf16_persist_kernel(GemmB16Args a, int m_blocks) {
+  constexpr int TM = 4, TN = 8;
+  extern __shared__ __attribute__((aligned(16))) unsigned char gp_smem[];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int g = lane >> 4, j = lane & 15;
+  const int wm = wave >> 1, wn = wave & 1;  // rows 64 wm .., features 128 wn ..
+  float* const sbias = reinterpret_cast<float*>(gp_smem + 2 * GP_STAGE + 8 * GP_EPI);
+  for (int c = tid; c < a.N; c += 512) sbias[c] = a.bias ? a.bias[c] : 0.0f;
+  __syncthreads();
+
+  // Tiles: XCD x (blocks x, x + 8, ..) takes the m blocks x per .. x per +
+  // per - 1, features fastest, so that the tiles in flight on an XCD share
+  // activation rows and weights in its L2.
+  const int nb = a.N / 256, per = (m_blocks + 7) / 8;
+  const int x0 = (blockIdx.x & 7) * per;
+  const int n_tiles = max(0, min(per, m_blocks - x0)) * nb;  // of this XCD
+  const int step = gridDim.x / 8;
+  const int n_st = a.K / 64;
+
+  // copies: copy i of a wave fills rows 32 wave + 8 i .. + 7 of a stage's
+  // activations and of its weights
+  const int crow = 32 * wave + (lane >> 3), cchunk = ((lane & 7) ^ (lane >> 3)) * 16;
+  const int woff = (lane >> 3) * a.ldw * 2 + cchunk;
+  auto tile_at = [&](int t) {
+    GpTile T;
+    T.m = (x0 + t / nb) * 256;
+    T.n = (t % nb) * 256;
+    T.x = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(a.X) + (size_t)T.m * a.ldx,
+                                            (short)0, -1, 0x00027000);
+    T.w = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<uint16_t*>(a.W) + (size_t)(T.n + 32 * wave) * a.ldw, (short)0, -1, 0x00027000);
+    return T;
+  };
+  auto copy = [&](const GpTile& T, int st, int slot) {
+    unsigned char* const base = gp_smem + slot * GP_STAGE + wave * 4096;
+    const int last = a.M - 1 - T.m;  // rows past M repeat the last one
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(
+          T.x, (__attribute__((address_space(3))) void*)(base + i * 1024), 16,
+          min(crow + 8 * i, last) * a.ldx * 2 + cchunk, st * 128, 0, 0);
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(
+          T.w, (__attribute__((address_space(3))) void*)(base + 32768 + i * 1024), 16, woff,
+          st * 128 + i * 16 * a.ldw, 0, 0);
+  };
+  // fragments of k-step ks: rows 64 wm + 16 p + j (128 wn + 16 q + j of the
+  // weights), chunk 4 ks + g
+  const uint32_t lds0 = lds_addr(gp_smem);
+  uint32_t xfrag[2], wfrag[2];
+#pragma unroll
+  for (int ks = 0; ks < 2; ++ks) {
+    const uint32_t s = j * 128 + ((4 * ks + g) ^ (j & 7)) * 16;
+    xfrag[ks] = lds0 + wm * 8192 + s;
+    wfrag[ks] = lds0 + 32768 + wn * 16384 + s;
+  }
+
+  int t = blockIdx.x >> 3;
+  if (t >= n_tiles) return;  // the whole block
+  GpTile T = tile_at(t);
+  copy(T, 0, 0);
+  int slot = 0;
+  int pending = 0;  // accesses newer than the next stage's copies (0, 1, 16 or 17)
+  while (true) {
+    floatx4 acc[TM][TN];
+#pragma unroll
+    for (int p = 0; p < TM; ++p)
+#pragma unroll
+      for (int q = 0; q < TN; ++q) acc[p][q] = floatx4{0.f, 0.f, 0.f, 0.f};
+    const int t_next = t + step;
+    const bool more = t_next < n_tiles;
+    const GpTile Tn = more ? tile_at(t_next) : T;
+    // Wave 0 fetches a 64-row group of the next tile's activations into L2, a
+    // stage's 128-byte line per row and stage (a copy to LDS that nobody
+    // reads), where four or more blocks share those rows: the copies proper
+    // run one stage ahead, too late for HBM behind the stores (1.2 M x 1024,
+    // K = 256: 1009 -> 907 us; with one or two blocks a row the extra
+    // requests cost more than they save, K = 512, N = 256: 384 -> 521 us).
+    const bool ahead = more && wave == 0 && nb >= 4 && T.n < 4 * 256;
+    const int poff = min(64 * (T.n / 256) + lane, a.M - 1 - Tn.m) * a.ldx * 2;
+    for (int st = 0; st < n_st; ++st, slot ^= 1) {
+      // this wave's copies of the stage have landed (newer are only the last
+      // epilogue's 16 stores and the fetch ahead), then everyone's
+      switch (pending) {
+        case 17: asm volatile("s_waitcnt vmcnt(17)" ::: "memory"); break;
+        case 16: asm volatile("s_waitcnt vmcnt(16)" ::: "memory"); break;
+        case 1: asm volatile("s_waitcnt vmcnt(1)" ::: "memory"); break;
+        default: asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      }
+      pending = 0;
+      lds_barrier();  // and everyone is past the other slot's reads
+      if (st + 1 < n_st) copy(T, st + 1, slot ^ 1);
+      else if (more) copy(Tn, 0, slot ^ 1);
+      if (ahead) {
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(
+            Tn.x, (__attribute__((address_space(3))) void*)(gp_smem + GP_LDS - 256), 4, poff,
+            st * 128, 0, 0);
+        pending = 1;
+      }
+      const uint32_t so = (uint32_t)slot * GP_STAGE;
+      const uint32_t xa[2] = {xfrag[0] + so, xfrag[1] + so}, wa[2] = {wfrag[0] + so, wfrag[1] + so};
+      lds_u32x4 xf[2][TM], f[2][2];
+      auto read_x = [&](auto KS) {
+        constexpr int ks = decltype(KS)::value;
+        xf[ks][0] = lds_read128_at<0>(xa[ks]);
+        xf[ks][1] = lds_read128_at<2048>(xa[ks]);
+        xf[ks][2] = lds_read128_at<4096>(xa[ks]);
+        xf[ks][3] = lds_read128_at<6144>(xa[ks]);
+      };
+      auto read_w = [&](auto H) {  // feature tiles 2 (H % 4) and the next of k-step H / 4
+        constexpr int h = decltype(H)::value;
+        f[h & 1][0] = lds_read128_at<(2 * (h & 3)) * 2048>(wa[h >> 2]);
+        f[h & 1][1] = lds_read128_at<(2 * (h & 3) + 1) * 2048>(wa[h >> 2]);
+      };
+      auto part = [&](auto H) {
+        constexpr int h = decltype(H)::value, q0 = 2 * (h & 3), b = h & 1, ks = h >> 2;
+        if constexpr (h == 2) read_x(std::integral_constant<int, 1>{});
+        if constexpr (h < 7) read_w(std::integral_constant<int, h + 1>{});
+        if constexpr (h == 0)
+          asm volatile("s_waitcnt lgkmcnt(2)"
+                       : "+v"(f[b][0]), "+v"(f[b][1]), "+v"(xf[0][0]), "+v"(xf[0][1]),
+                         "+v"(xf[0][2]), "+v"(xf[0][3])::"memory");
+        else if constexpr (h == 2)
+          asm volatile("s_waitcnt lgkmcnt(6)" : "+v"(f[b][0]), "+v"(f[b][1])::"memory");
+        else if constexpr (h == 4)
+          asm volatile("s_waitcnt lgkmcnt(2)"
+                       : "+v"(f[b][0]), "+v"(f[b][1]), "+v"(xf[1][0]), "+v"(xf[1][1]),
+                         "+v"(xf[1][2]), "+v"(xf[1][3])::"memory");
+        else if constexpr (h == 7)
+          asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(f[b][0]), "+v"(f[b][1])::"memory");
+        else
+          asm volatile("s_waitcnt lgkmcnt(2)" : "+v"(f[b][0]), "+v"(f[b][1])::"memory");
+#pragma unroll
+        for (int p = 0; p < TM; ++p)
+#pragma unroll
+          for (int q = 0; q < 2; ++q)
+            acc[p][q0 + q] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                __builtin_bit_cast(bf16x8, f[b][q]), __builtin_bit_cast(bf16x8, xf[ks][p]),
+                acc[p][q0 + q], 0, 0, 0);
+      };
+      read_x(std::integral_constant<int, 0>{});
+      read_w(std::integral_constant<int, 0>{});
+      part(std::integral_constant<int, 0>{});
+      part(std::integral_constant<int, 1>{});
+      part(std::integral_constant<int, 2>{});
+      part(std::integral_constant<int, 3>{});
+      part(std::integral_constant<int, 4>{});
+      part(std::integral_constant<int, 5>{});
+      part(std::integral_constant<int, 6>{});
+      part(std::integral_constant<int, 7>{});
+    }
+
+    // Epilogue, per wave without barriers, its LDS accesses outside the
+    // compiler's view (it would wait for the next tile's copies).  A group of
+    // 16 rows x 128 bytes goes to the wave's 2 KB with chunk c of row r at
+    // slot c ^ (r & 7) and comes back eight lanes a row, two 8-row reads.
+    const uint32_t epi = lds0 + 2 * GP_STAGE + wave * GP_EPI;
+    const uint32_t bat = lds_addr(sbias) + (T.n + 128 * wn + 4 * g) * 4;
+    const int m0 = T.m + 64 * wm, n0 = T.n + 128 * wn;
+    const int er = lane >> 3, ec = lane & 7;  // row and chunk of a read
+    const uint32_t erd = epi + er * 128 + ((ec ^ er) * 16);  // rows er and er + 8: the same slot
+    const bool full = T.m + 256 <= a.M;
+    auto act = [&](float v, float b) {
+      float t = v + b;
+      if (ACT == ACT_GELU) t = gelu<MATH_HW>(t);
+      else if (ACT == ACT_RELU) t = fmaxf(0.0f, t);
+      return t;
+    };
+    if constexpr (!F32) {
+#pragma unroll
+      for (int half = 0; half < 2; ++half) {  // features 64 half .. of the wave's 128
+        lds_u32x4 bv[4];
+        bv[0] = half ? lds_read128_at<256>(bat) : lds_read128_at<0>(bat);
+        bv[1] = half ? lds_read128_at<320>(bat) : lds_read128_at<64>(bat);
+        bv[2] = half ? lds_read128_at<384>(bat) : lds_read128_at<128>(bat);
+        bv[3] = half ? lds_read128_at<448>(bat) : lds_read128_at<192>(bat);
+        lds_wait4(bv[0], bv[1], bv[2], bv[3]);
+#pragma unroll
+        for (int p = 0; p < TM; ++p) {
+#pragma unroll
+          for (int q = 0; q < 4; ++q) {
+            const floatx4 c = acc[p][4 * half + q];
+            const uint32_t lo =
+                (uint32_t)f32_to_bf16(act(c[0], u2f(bv[q][0]))) |
+                ((uint32_t)f32_to_bf16(act(c[1], u2f(bv[q][1]))) << 16);
+            const uint32_t hi =
+                (uint32_t)f32_to_bf16(act(c[2], u2f(bv[q][2]))) |
+                ((uint32_t)f32_to_bf16(act(c[3], u2f(bv[q][3]))) << 16);
+            lds_write64_at<0>(epi + j * 128 + (((2 * q + (g >> 1)) ^ (j & 7)) * 16) + (g & 1) * 8,
+                              lo, hi);
+          }
+          lds_u32x4 v0 = lds_read128_at<0>(erd), v1 = lds_read128_at<1024>(erd);
+          asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(v0), "+v"(v1)::"memory");
+          uint16_t* const o =
+              reinterpret_cast<uint16_t*>(a.C) + (size_t)(m0 + 16 * p + er) * a.ldc + n0 + 64 * half + 8 * ec;
+          if (full || m0 + 16 * p + er < a.M) *reinterpret_cast<lds_u32x4*>(o) = v0;
+          if (full || m0 + 16 * p + er + 8 < a.M)
+            *reinterpret_cast<lds_u32x4*>(o + (size_t)8 * a.ldc) = v1;
+        }
+      }
+      pending = full ? pending + 16 : 0;
+    } else {
+      pending = 0;
+#pragma unroll
+      for (int qq = 0; qq < 4; ++qq) {  // features 32 qq .. of the wave's 128
+        lds_u32x4 bv[2];
+        bv[0] = qq == 0 ? lds_read128_at<0>(bat) : qq == 1 ? lds_read128_at<128>(bat)
+              : qq == 2 ? lds_read128_at<256>(bat) : lds_read128_at<384>(bat);
+        bv[1] = qq == 0 ? lds_read128_at<64>(bat) : qq == 1 ? lds_read128_at<192>(bat)
+              : qq == 2 ? lds_read128_at<320>(bat) : lds_read128_at<448>(bat);
+        asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(bv[0]), "+v"(bv[1])::"memory");
+        float4 rs[TM][2];
+        if (a.res) {
+#pragma unroll
+          for (int p = 0; p < TM; ++p)
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+              const int m = min(m0 + 16 * p + er + 8 * h, a.M - 1);
+              rs[p][h] = *reinterpret_cast<const float4*>(a.res + (size_t)m * a.ldr + n0 + 32 * qq + 4 * ec);
+            }
+        }
+#pragma unroll
+        for (int p = 0; p < TM; ++p) {
+#pragma unroll
+          for (int q = 0; q < 2; ++q) {
+            const floatx4 c = acc[p][2 * qq + q];
+            lds_u32x4 v;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) v[e] = f2u(act(c[e], u2f(bv[q][e])));
+            lds_write128_at<0>(epi + j * 128 + (((4 * q + g) ^ (j & 7)) * 16), v);
+          }
+          lds_u32x4 v[2];
+          v[0] = lds_read128_at<0>(erd);
+          v[1] = lds_read128_at<1024>(erd);
+          asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(v[0]), "+v"(v[1])::"memory");
+#pragma unroll
+          for (int h = 0; h < 2; ++h) {
+            const int m = m0 + 16 * p + er + 8 * h;
+            float4 o = make_float4(u2f(v[h][0]), u2f(v[h][1]), u2f(v[h][2]), u2f(v[h][3]));
+            if (a.res) {
+              const float4 e = rs[p][h];
+              o = make_float4(o.x + e.x, o.y + e.y, o.z + e.z, o.w + e.w);
+            }
+            if (full || m < a.M) {
+              const size_t at = (size_t)m * a.ldc + n0 + 32 * qq + 4 * ec;
+              *reinterpret_cast<float4*>(reinterpret_cast<float*>(a.C) + at) = o;
+              if (a.C2)
+                *reinterpret_cast<ushort4*>(a.C2 + at) = make_ushort4(
+                    f32_to_bf16(o.x), f32_to_bf16(o.y), f32_to_bf16(o.z), f32_to_bf16(o.w));
+            }
+          }
+        }
+      }
+    }
+    if (!more) break;
+    t = t_next;
+    T = Tn;
+  }
+}
+
+// What the kernel's addressing takes: whole 256-feature tiles up to
+// GP_MAX_N, whole 64-k stages, 16-byte rows, a tile's rows within 32-bit byte
+// offsets; a residual or a bf16 copy only beside fp32 output.
+static bool b16_persist_fits(const GemmB16Args& a) {
+  return a.N % 256 == 0 && a.N <= GP_MAX_N && a.K % 64 == 0 && a.K >= 64 && a.ldx % 8 == 0 &&
+         a.ldw % 8 == 0 && a.ldw >= a.K && a.ldx <= (1 << 20) && a.ldw <= (1 << 20) &&
+         a.ldc % 8 == 0 && (!a.res || a.ldr % 4 == 0) && (!a.c_bf16 || (!a.res && !a.C2));
+}
+
+static hipError_t launch_b16_persist(const GemmB16Args& a, hipStream_t s) {
+  const int m_blocks = (int)(((long long)a.M + 255) / 256);
+  // a multiple of eight blocks (one share of the XCDs each), at most one per CU
+  const long long tiles = (long long)((m_blocks + 7) / 8) * (a.N / 256) * 8;
+  const unsigned grid = (unsigned)std::min<long long>(tiles, 256);
+#define BOA_B16_ONE(ACTv, F)                                                                    \
+  {                                                                                             \
+    static const hipError_t attr =                                                              \
+        hipFuncSetAttribute(reinterpret_cast<const void*>(gemm_bf16_persist_kernel<ACTv, F>),   \
+                            hipFuncAttributeMaxDynamicSharedMemorySize, GP_LDS);                \
+    if (attr != hipSuccess) return attr;                                                        \
+    BOA_LAUNCH((gemm_bf16_persist_kernel<ACTv, F>), dim3(grid), dim3(512), GP_LDS, s, a,        \
+               m_blocks);                                                                       \
+  }
+#define BOA_B16_GO(ACTv)                    \
+  if (a.c_bf16) BOA_B16_ONE(ACTv, false)    \
+  else BOA_B16_ONE(ACTv, true)
+  switch (a.act) {
+    case ACT_NONE: BOA_B16_GO(ACT_NONE) break;
+    case ACT_GELU: BOA_B16_GO(ACT_GELU) break;
+    case ACT_RELU: BOA_B16_GO(ACT_RELU) break;
+    default: return hipErrorInvalidValue;
+  }
+#undef BOA_B16_GO
+#undef BOA_B16_ONE
+  return hipGetLastError();
+}
+
 // W must hold round_up(N, 256) rows (zero padded) for every configuration.
-// Chosen from sweeps on MI355X at compress shapes (M ~ 10^6): 256x256 with
-// 16 waves of 64x64 (the LDS traffic per MFMA halves against 32x64 waves) for
-// N >= 256 -- one LDS stage where K or N is at least 512 (3-8 % faster
-// there), two for the 256x256 head GEMMs -- and 128x64 with 8 waves for the
-// narrow x_proj.  Smaller tiles (128x128, 8-wave 256x256) were 25-45 %
-// slower.
+// Outputs of whole 256-feature tiles run on the persistent blocks (TFLOP/s at
+// M about 10^6, against the 256 x 256 blocks of gemm_bf16_kernel: K 256 N
+// 1024 435 -> 694, K 512 N 256 594 -> 819, K 512 N 2048 667 -> 946, K 1024 N
+// 512 799 -> 1064, K 2048 N 512 with residual 657 -> 855, GELU K 512 N 2048
+// 540 -> 731; M 255 to 1300 as fast or faster); narrower or unaligned ones
+// (x_proj, d_model 64's and 128's narrow outputs) on 128 x 64 blocks with 8
+// waves.
 hipError_t gemm_bf16(const GemmB16Args& a, hipStream_t s) {
   if (a.M <= 0 || a.N <= 0) return hipSuccess;
-  if (a.N >= 256 && (a.N >= 512 || a.K >= 512)) return launch_b16<256, 256, 4, 4, 64, 1>(a, s);
-  if (a.N >= 256) return launch_b16<256, 256, 4, 4, 64>(a, s);
+  if (b16_persist_fits(a)) return launch_b16_persist(a, s);
   return launch_b16<128, 64, 4, 2, 64>(a, s);
 }
 
