@@ -112,10 +112,18 @@ __device__ __forceinline__ lds_u32x4 lds_read128_at(uint32_t a) {
   asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(v) : "v"(a), "n"(OFF) : "memory");
   return v;
 }
+// two dwords, at a + 256 O0 and a + 256 O1
+typedef uint32_t lds_u32x2 __attribute__((ext_vector_type(2)));
+template <int O0, int O1>
+__device__ __forceinline__ lds_u32x2 lds_read2_at(uint32_t a) {
+  lds_u32x2 v;
+  asm volatile("ds_read2st64_b32 %0, %1 offset0:%2 offset1:%3"
+               : "=v"(v) : "v"(a), "n"(O0), "n"(O1) : "memory");
+  return v;
+}
 template <int OFF>
 __device__ __forceinline__ void lds_write64_at(uint32_t a, uint32_t lo, uint32_t hi) {
-  typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
-  const u32x2 v = {lo, hi};
+  const lds_u32x2 v = {lo, hi};
   asm volatile("ds_write_b64 %0, %1 offset:%2" ::"v"(a), "v"(v), "n"(OFF) : "memory");
 }
 template <int OFF>

@@ -18,6 +18,10 @@
 // accumulators are 4 consecutive n of one row m and the epilogue stores a
 // float4 per lane.  LDS: activations [BM][BK+4] (16-byte rows for b128
 // stores), weights [BK][BN+16]; both double-buffered, one barrier per K step.
+#include <algorithm>
+#include <type_traits>
+
+#include "block_device.h"
 #include "boa_kernels.h"
 #include "coder_device.h"
 
@@ -296,6 +300,237 @@ void gemm_f32_kernel(
   }
 }
 
+// ------------------------------------------------------- persistent blocks
+// 256 rows x 256 features a tile, eight waves of 64 x 128 (two per SIMD), one
+// block per CU that walks over tiles.  fp32 MFMAs and vector instructions
+// share the SIMD's FMA units (they do not overlap, see boa_math.h), so the K
+// loop holds little but MFMAs: 32-k stages are copied straight to LDS (no
+// staging registers or LDS stores), most of an address is an instruction
+// offset, and a 4-k step's 32 MFMAs read 12 operand dwords with six LDS
+// instructions.  The loop runs at the MFMA rate (6.9 us a stage against 6.8);
+// what costs besides is the output (256 KB a tile in 25 us, every CU at the
+// same time, against 55 us of MFMAs at K = 256): the next tile's stages 0 and
+// 1 are copied ahead of the stores, which drain behind them.  Keeping half a
+// tile in registers and storing it between the next one's k-steps needed
+// more registers than there are (spills; with 64 x 64 waves, where it fits,
+// the loop took 11 % longer).
+// LDS: two 64 KB stages.  Activations: rows of 128 bytes, the 16-byte chunk
+// c of row r at slot c ^ ((r >> 1) & 7); weights: k rows of 1 KB, the 64-byte
+// group q of row k at slot q ^ (k & 3): the 64 lanes of an operand read fall
+// on the 64 banks either way.  Then the bias of every feature.
+struct GfTile {
+  __amdgpu_buffer_rsrc_t x, w;  // the tile's activation rows, its weight columns
+  int m, n;
+};
+constexpr int GF_X = 32768, GF_STAGE = 2 * GF_X, GF_MAX_N = 2048;
+constexpr int GF_LDS = 2 * GF_STAGE + 4 * GF_MAX_N;
+
+template <int ACT>
+__global__ __launch_bounds__(512, 2) void gemm_f32_persist_kernel(GemmArgs a, int m_blocks) {
+  constexpr int TM = 4, TN = 8;
+  extern __shared__ __attribute__((aligned(16))) unsigned char gf_smem[];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int g = lane >> 4, j = lane & 15;
+  const int wm = wave >> 1, wn = wave & 1;  // rows 64 wm .., features 128 wn ..
+  float* const sbias = reinterpret_cast<float*>(gf_smem + 2 * GF_STAGE);
+  for (int c = tid; c < a.N; c += 512) sbias[c] = a.bias ? a.bias[c] : 0.0f;
+  __syncthreads();
+
+  // Tiles: XCD x (blocks x, x + 8, ..) takes the m blocks x per .. x per +
+  // per - 1, features fastest, so that the tiles in flight on an XCD share
+  // activation rows and weights in its L2.
+  const int nb = a.N / 256, per = (m_blocks + 7) / 8;
+  const int x0 = (blockIdx.x & 7) * per;
+  const int n_tiles = max(0, min(per, m_blocks - x0)) * nb;  // of this XCD
+  const int step = gridDim.x / 8;
+  const int n_st = a.K / 32;
+
+  // copies: copy i of a wave fills rows 32 wave + 8 i .. + 7 of a stage's
+  // activations and k row 4 wave + i of its weights
+  const int xrow = (32 * wave + (lane >> 3)) * a.ldx * 4;
+  const int xoff[2] = {xrow + ((lane & 7) ^ (lane >> 4)) * 16,
+                       xrow + ((lane & 7) ^ (4 + (lane >> 4))) * 16};
+  auto tile_at = [&](int t) {
+    GfTile T;
+    // the last rows' tile starts early: rows that two tiles hold get the same
+    // values from both
+    T.m = min((x0 + t / nb) * 256, a.M - 256);
+    T.n = (t % nb) * 256;
+    T.x = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(a.X) + (size_t)T.m * a.ldx,
+                                            (short)0, -1, 0x00027000);
+    T.w = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(a.W) + T.n, (short)0, -1,
+                                            0x00027000);
+    return T;
+  };
+  auto copy_part = [&](const GfTile& T, int st, int slot, int i) {
+    unsigned char* const base = gf_smem + slot * GF_STAGE + wave * 4096 + i * 1024;
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(
+        T.x, (__attribute__((address_space(3))) void*)base, 16, xoff[i & 1],
+        st * 128 + 32 * i * a.ldx, 0, 0);
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(
+        T.w, (__attribute__((address_space(3))) void*)(base + GF_X), 16, (lane * 16) ^ (64 * i),
+        (st * 32 + 4 * wave + i) * a.ldw * 4, 0, 0);
+  };
+  auto copy = [&](const GfTile& T, int st, int slot) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) copy_part(T, st, slot, i);
+  };
+  // operand addresses: activations of 4-k step s at xat ^ 16 s (row tiles are
+  // instruction offsets), weights of feature tiles q and q + 4 at wat ^ 64 q
+  // (so are steps); the stages start at multiples of 128 bytes
+  const uint32_t lds0 = lds_addr(gf_smem);
+  const uint32_t xat = lds0 + wm * 8192 + j * 128 + ((j >> 1) & 7) * 16 + 4 * g;
+  const uint32_t wat = lds0 + GF_X + wn * 512 + g * 1024 + g * 64 + 4 * j;
+
+  int t = blockIdx.x >> 3;
+  if (t >= n_tiles) return;  // the whole block
+  GfTile T = tile_at(t);
+  copy(T, 0, 0);
+  copy(T, 1, 1);
+  int slot = 0;
+
+  bool stores = false;  // the last epilogue's 32 stores, behind copies 0 and 1
+  while (true) {
+    floatx4 acc[TM][TN];
+#pragma unroll
+    for (int p = 0; p < TM; ++p)
+#pragma unroll
+      for (int q = 0; q < TN; ++q) acc[p][q] = floatx4{0.f, 0.f, 0.f, 0.f};
+    const int t_next = t + step;
+    const bool more = t_next < n_tiles;
+    const GfTile Tn = more ? tile_at(t_next) : T;
+    for (int st = 0; st < n_st; ++st, slot ^= 1) {
+      // this wave's copies of the stage have landed (newer may be, at stage 0,
+      // the eight copies of stage 1 and the stores, at stage 1 those), then
+      // everyone's
+      if (st == 0) {
+        if (stores) asm volatile("s_waitcnt vmcnt(40)" ::: "memory");
+        else asm volatile("s_waitcnt vmcnt(8)" ::: "memory");
+      } else if (st == 1 && stores) {
+        asm volatile("s_waitcnt vmcnt(32)" ::: "memory");
+      } else {
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      }
+      lds_barrier();  // and everyone is past the other slot's reads
+      const bool here = st + 1 < n_st, copying = st > 0 && (here || more);
+      const GfTile& Tc = here ? T : Tn;
+      const int stc = here ? st + 1 : 0;
+      const uint32_t so = (uint32_t)slot * GF_STAGE;
+      const uint32_t wa = wat + so, xa = xat + so;
+      lds_u32x2 xf[2][2], wf[2][4];
+      auto read = [&](auto S) {
+        constexpr int s = decltype(S)::value, b = s & 1;
+        const uint32_t x = xa ^ (16 * s);
+        xf[b][0] = lds_read2_at<0, 8>(x);    // row tiles 0, 1
+        xf[b][1] = lds_read2_at<16, 24>(x);  // 2, 3
+        wf[b][0] = lds_read2_at<16 * s, 16 * s + 1>(wa);  // feature tiles 0, 4
+        wf[b][1] = lds_read2_at<16 * s, 16 * s + 1>(wa ^ 64);
+        wf[b][2] = lds_read2_at<16 * s, 16 * s + 1>(wa ^ 128);
+        wf[b][3] = lds_read2_at<16 * s, 16 * s + 1>(wa ^ 192);
+      };
+      auto kstep = [&](auto S) {
+        constexpr int s = decltype(S)::value, b = s & 1;
+        // the next step's operands are read while this one multiplies
+        if constexpr (s < 7) read(std::integral_constant<int, s + 1>{});
+        asm volatile("s_waitcnt lgkmcnt(%6)"
+                     : "+v"(xf[b][0]), "+v"(xf[b][1]), "+v"(wf[b][0]), "+v"(wf[b][1]),
+                       "+v"(wf[b][2]), "+v"(wf[b][3])
+                     : "n"(s < 7 ? 6 : 0)
+                     : "memory");
+        if constexpr (s < 4)
+          if (copying) copy_part(Tc, stc, slot ^ 1, s);
+#pragma unroll
+        for (int q = 0; q < TN; ++q)
+#pragma unroll
+          for (int p = 0; p < TM; ++p)
+            acc[p][q] = __builtin_amdgcn_mfma_f32_16x16x4f32(
+                u2f(wf[b][q & 3][q >> 2]), u2f(xf[b][p >> 1][p & 1]), acc[p][q], 0, 0, 0);
+      };
+      read(std::integral_constant<int, 0>{});
+      kstep(std::integral_constant<int, 0>{});
+      kstep(std::integral_constant<int, 1>{});
+      kstep(std::integral_constant<int, 2>{});
+      kstep(std::integral_constant<int, 3>{});
+      kstep(std::integral_constant<int, 4>{});
+      kstep(std::integral_constant<int, 5>{});
+      kstep(std::integral_constant<int, 6>{});
+      kstep(std::integral_constant<int, 7>{});
+    }
+
+    // the tile's values: lane (g, j) has features n0 + 16 q .. + 3 of rows
+    // m0 + 16 p, stored in 64-byte pieces
+    if (more) {
+      lds_barrier();  // everyone is past the last stage's reads
+      copy(Tn, 1, slot ^ 1);
+    }
+    const uint32_t bat = lds_addr(sbias) + (T.n + 128 * wn + 4 * g) * 4;
+    const int m0 = T.m + 64 * wm + j, n0 = T.n + 128 * wn + 4 * g;
+    auto feature_tile = [&](auto Q) {
+      constexpr int q = decltype(Q)::value;
+      lds_u32x4 bv = lds_read128_at<64 * q>(bat);
+      asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(bv)::"memory");
+#pragma unroll
+      for (int p = 0; p < TM; ++p) {
+        floatx4 v;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          float x = acc[p][q][e] + u2f(bv[e]);
+          if (ACT == ACT_GELU) x = gelu(x);
+          else if (ACT == ACT_RELU) x = fmaxf(0.0f, x);
+          v[e] = x;
+        }
+        *reinterpret_cast<floatx4*>(a.C + (size_t)(m0 + 16 * p) * a.ldc + n0 + 16 * q) = v;
+      }
+    };
+    feature_tile(std::integral_constant<int, 0>{});
+    feature_tile(std::integral_constant<int, 1>{});
+    feature_tile(std::integral_constant<int, 2>{});
+    feature_tile(std::integral_constant<int, 3>{});
+    feature_tile(std::integral_constant<int, 4>{});
+    feature_tile(std::integral_constant<int, 5>{});
+    feature_tile(std::integral_constant<int, 6>{});
+    feature_tile(std::integral_constant<int, 7>{});
+    stores = true;
+    if (!more) break;
+    t = t_next;
+    T = Tn;
+  }
+}
+
+// What the kernel's addressing takes: whole 256-feature tiles up to GF_MAX_N,
+// whole 32-k stages (two at least), 16-byte rows, a tile's rows and the
+// weights within 32-bit byte offsets, a tile's worth of rows, no residual.
+static bool f32_persist_fits(const GemmArgs& a) {
+  return a.N % 256 == 0 && a.N <= GF_MAX_N && a.K % 32 == 0 && a.K >= 64 && a.ldx % 4 == 0 &&
+         a.ldw % 4 == 0 && a.ldw >= a.N && a.ldx <= (1 << 20) &&
+         (long long)a.K * a.ldw < (1 << 28) && a.ldc % 4 == 0 && !a.res && a.M >= 256 &&
+         a.X != a.C;
+}
+
+// Whether the tiles fill the CUs in whole rounds (one block per CU; the 32
+// blocks of an XCD share its m blocks): at 70 % of 3 rounds (17,000 x 2048)
+// the 128 x 256 blocks, finer and two per CU, were 11 % faster, at 50 % 24 %.
+static bool f32_persist_fills(const GemmArgs& a) {
+  const long long mb = (a.M + 255) / 256, nb = a.N / 256;
+  const long long rounds = ((mb + 7) / 8 * nb + 31) / 32;
+  return 100 * mb * nb >= 85 * 256 * rounds;
+}
+
+template <int ACT>
+static hipError_t f32_persist_go(const GemmArgs& a, hipStream_t s) {
+  static const hipError_t attr =
+      hipFuncSetAttribute(reinterpret_cast<const void*>(gemm_f32_persist_kernel<ACT>),
+                          hipFuncAttributeMaxDynamicSharedMemorySize, GF_LDS);
+  if (attr != hipSuccess) return attr;
+  const int m_blocks = (int)(((long long)a.M + 255) / 256);
+  // a multiple of eight blocks (one share of the XCDs each), at most one per CU
+  const long long tiles = (long long)((m_blocks + 7) / 8) * (a.N / 256) * 8;
+  const unsigned grid = (unsigned)std::min<long long>(tiles, 256);
+  BOA_LAUNCH((gemm_f32_persist_kernel<ACT>), dim3(grid), dim3(512), GF_LDS, s, a, m_blocks);
+  return hipGetLastError();
+}
+
 template <int BM, int BN, int WM_, int WN_, int BK>
 static hipError_t launch_cfg(const GemmArgs& a, hipStream_t s, int swizzle = 1) {
   if (a.K % BK || a.ldw < (a.N + BN - 1) / BN * BN) return hipErrorInvalidValue;
@@ -318,9 +553,13 @@ static hipError_t launch_cfg(const GemmArgs& a, hipStream_t s, int swizzle = 1) 
 }
 
 // Tile choice only changes the schedule, never the numerics (see above).
-// Chosen from a sweep on MI355X (fp32 MFMA): many waves per CU matter more
-// than register blocking.  Large M (a compress tile): 128x256 with 16 waves
-// (32x64 each) for N >= 256, 128x64 with 8 waves for the narrow x_proj;
+// Large M (a compress tile), N >= 256: persistent 256x256 blocks where the
+// shape fits them (TFLOP/s at 1.6 M rows, against 128x256 blocks of 16 waves:
+// K 256 N 1024 113.5 -> 126.6, with GELU at 400,000 rows 98.6 -> 105.9), the
+// 128x256 blocks otherwise (the LayerNorm epilogues and FF2's residual, 256
+// wide: equal to 2 % at whole rounds of the CUs, slower between, and their
+// epilogues overlap the other resident block's MFMAs); 128x64 with 8 waves for
+// the narrow x_proj;
 // small M (a decode step, M = lanes): 32x32 with four 16x16 waves and BK=32.
 int gemm_f32_config(const GemmArgs& a) {
   if (a.M >= 16384) return a.N >= 256 ? 0 : 1;
@@ -369,7 +608,16 @@ hipError_t gemm_f32(const GemmArgs& a, hipStream_t s) {
   if (a.M <= 0 || a.N <= 0) return hipSuccess;
   if (a.K % 16 != 0 || a.ldx % 4 != 0 || a.ldw % 4 != 0) return hipErrorInvalidValue;
   switch (gemm_f32_config(a)) {
-    case 0: return launch_cfg<128, 256, 4, 4, 16>(a, s);
+    case 0:
+      if (f32_persist_fits(a) && f32_persist_fills(a)) {
+        switch (a.act) {
+          case ACT_NONE: return f32_persist_go<ACT_NONE>(a, s);
+          case ACT_GELU: return f32_persist_go<ACT_GELU>(a, s);
+          case ACT_RELU: return f32_persist_go<ACT_RELU>(a, s);
+          default: return hipErrorInvalidValue;
+        }
+      }
+      return launch_cfg<128, 256, 4, 4, 16>(a, s);
     case 1: return launch_cfg<128, 64, 4, 2, 16>(a, s);
     default:
       return a.K % 32 == 0 ? launch_cfg<32, 32, 2, 2, 32>(a, s) : launch_cfg<32, 32, 2, 2, 16>(a, s);

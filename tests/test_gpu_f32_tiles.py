@@ -1,0 +1,34 @@
+"""fp32 compress GEMM tiles: from 16,384 rows on the plain GEMMs of 256-wide
+outputs run in 256-row persistent blocks, whose last tile starts early when
+the rows are no multiple of 256, where those tiles fill the CUs.  The row
+counts here are whole rounds of the CUs with 0, 1 and 255 rows over a tile.  The logits of every
+row equal those of short calls (other kernels), and the rows past the last
+one stay untouched."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("d,rows", [(64, 65281), (64, 65535), (256, 16384), (256, 65281),
+                                    (256, 65535), (512, 65535)])
+def test_rows_around_tiles(make_weights, d, rows):
+    import torch
+
+    import boa_hip
+    c = boa_hip.Codec(d, 1, 16, rows)
+    c.set_stream(torch.cuda.current_stream().cuda_stream)
+    c.load_weights(make_weights(d, 1))
+    tok = torch.from_numpy(np.random.default_rng(d).integers(0, 256, rows, dtype=np.uint8)).cuda()
+    c.reset_state(rows)
+    got = torch.full((rows + 300, 256), -7.0, device="cuda")
+    c.forward_chunk(tok, rows, 1, got)
+    want = torch.zeros((rows, 256), device="cuda")
+    for r in range(0, rows, 8192):
+        n = min(8192, rows - r)
+        c.reset_state(n)
+        c.forward_chunk(tok[r:r + n].contiguous(), n, 1, want[r:r + n])
+    torch.cuda.synchronize()
+    assert bool((got[rows:] == -7.0).all())
+    assert torch.equal(got[:rows].view(torch.int32), want.view(torch.int32))
+    c.close()
