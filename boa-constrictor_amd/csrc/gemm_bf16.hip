@@ -289,7 +289,7 @@ struct GpTile {
 template <int ACT, bool F32>
 __global__ __launch_bounds__(512, 2) void gemm_bf16_persist_kernel(GemmB16Args a, int m_blocks) {
   constexpr int TM = 4, TN = 8;
-  extern __shared__ __attribute__((aligned(16))) unsigned char gp_smem[];
+  __shared__ __attribute__((aligned(16))) unsigned char gp_smem[GP_LDS];
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int g = lane >> 4, j = lane & 15;
@@ -563,26 +563,19 @@ static hipError_t launch_b16_persist(const GemmB16Args& a, hipStream_t s) {
   // a multiple of eight blocks (one share of the XCDs each), at most one per CU
   const long long tiles = (long long)((m_blocks + 7) / 8) * (a.N / 256) * 8;
   const unsigned grid = (unsigned)std::min<long long>(tiles, 256);
-#define BOA_B16_ONE(ACTv, F)                                                                    \
-  {                                                                                             \
-    static const hipError_t attr =                                                              \
-        hipFuncSetAttribute(reinterpret_cast<const void*>(gemm_bf16_persist_kernel<ACTv, F>),   \
-                            hipFuncAttributeMaxDynamicSharedMemorySize, GP_LDS);                \
-    if (attr != hipSuccess) return attr;                                                        \
-    BOA_LAUNCH((gemm_bf16_persist_kernel<ACTv, F>), dim3(grid), dim3(512), GP_LDS, s, a,        \
-               m_blocks);                                                                       \
-  }
-#define BOA_B16_GO(ACTv)                    \
-  if (a.c_bf16) BOA_B16_ONE(ACTv, false)    \
-  else BOA_B16_ONE(ACTv, true)
+#define BOA_B16_GO(ACTv)                                                                       \
+  if (a.c_bf16)                                                                                \
+    BOA_LAUNCH((gemm_bf16_persist_kernel<ACTv, false>), dim3(grid), dim3(512), 0, s, a,        \
+               m_blocks);                                                                      \
+  else                                                                                         \
+    BOA_LAUNCH((gemm_bf16_persist_kernel<ACTv, true>), dim3(grid), dim3(512), 0, s, a, m_blocks)
   switch (a.act) {
-    case ACT_NONE: BOA_B16_GO(ACT_NONE) break;
-    case ACT_GELU: BOA_B16_GO(ACT_GELU) break;
-    case ACT_RELU: BOA_B16_GO(ACT_RELU) break;
+    case ACT_NONE: BOA_B16_GO(ACT_NONE); break;
+    case ACT_GELU: BOA_B16_GO(ACT_GELU); break;
+    case ACT_RELU: BOA_B16_GO(ACT_RELU); break;
     default: return hipErrorInvalidValue;
   }
 #undef BOA_B16_GO
-#undef BOA_B16_ONE
   return hipGetLastError();
 }
 

@@ -328,7 +328,7 @@ constexpr int GF_LDS = 2 * GF_STAGE + 4 * GF_MAX_N;
 template <int ACT>
 __global__ __launch_bounds__(512, 2) void gemm_f32_persist_kernel(GemmArgs a, int m_blocks) {
   constexpr int TM = 4, TN = 8;
-  extern __shared__ __attribute__((aligned(16))) unsigned char gf_smem[];
+  __shared__ __attribute__((aligned(16))) unsigned char gf_smem[GF_LDS];
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int g = lane >> 4, j = lane & 15;
@@ -519,15 +519,11 @@ static bool f32_persist_fills(const GemmArgs& a) {
 
 template <int ACT>
 static hipError_t f32_persist_go(const GemmArgs& a, hipStream_t s) {
-  static const hipError_t attr =
-      hipFuncSetAttribute(reinterpret_cast<const void*>(gemm_f32_persist_kernel<ACT>),
-                          hipFuncAttributeMaxDynamicSharedMemorySize, GF_LDS);
-  if (attr != hipSuccess) return attr;
   const int m_blocks = (int)(((long long)a.M + 255) / 256);
   // a multiple of eight blocks (one share of the XCDs each), at most one per CU
   const long long tiles = (long long)((m_blocks + 7) / 8) * (a.N / 256) * 8;
   const unsigned grid = (unsigned)std::min<long long>(tiles, 256);
-  BOA_LAUNCH((gemm_f32_persist_kernel<ACT>), dim3(grid), dim3(512), GF_LDS, s, a, m_blocks);
+  BOA_LAUNCH((gemm_f32_persist_kernel<ACT>), dim3(grid), dim3(512), 0, s, a, m_blocks);
   return hipGetLastError();
 }
 
