@@ -85,8 +85,9 @@ struct LnEpi {
   int n;     // the LayerNorm's width (real features of the 256)
 };
 hipError_t gemm_f32_ln(const GemmArgs& a, const LnEpi& ln, hipStream_t s);
-// Tile configuration gemm_f32 picks: 0 = 128x256 (bulk GEMMs of a compress
-// tile), 1 = 128x64 (narrow compress GEMMs), 2 = 32x32 (decode-step sizes).
+// Tile configuration gemm_f32 picks where the persistent blocks do not take
+// the shape: 0 = 128x256 (bulk GEMMs of a compress tile), 1 = 128x64 (narrow
+// compress GEMMs, some thousand rows), 3 = 64x32, 2 = 32x32 (decode-step sizes).
 int gemm_f32_config(const GemmArgs& a);
 
 // Encoder / decoder coder state (layout of RCState / RCDecState,

@@ -555,10 +555,24 @@ static hipError_t launch_cfg(const GemmArgs& a, hipStream_t s, int swizzle = 1) 
 // 128x256 blocks otherwise (the LayerNorm epilogues and FF2's residual, 256
 // wide: equal to 2 % at whole rounds of the CUs, slower between, and their
 // epilogues overlap the other resident block's MFMAs); 128x64 with 8 waves for
-// the narrow x_proj;
-// small M (a decode step, M = lanes): 32x32 with four 16x16 waves and BK=32.
+// the narrow x_proj.
+// Fewer rows (a forward call of some thousand tokens): 128x64 blocks from
+// about three rounds of the CUs (700 blocks) on, 64x32 blocks of eight waves
+// from two rounds (500) on, else 32x32 with four waves, whose finer tiles fill
+// more CUs.  µs of 128x64 / 64x32 / 32x32 at 8103 rows: N 1024 K 256 46.3 /
+// 49.3 / 51.6, N 256 K 512 29.7 / 27.8 / 32.5, N 256 K 1024 53.4 / 48.7 /
+// 60.0, N 2048 K 512 153.9 / 179.4 / 197.4; beside the lines, N 1024 K 256:
+// 6000 rows (752 and 3008 blocks) 37.3 / 38.6 / 39.5, 4000 rows (512, 2016)
+// 27.8 / 27.1 / 28.6, 1000 rows (128, 512) 16.5 / 10.1 / 10.2; N 256 K 512:
+// 4000 rows (128, 504) 27.8 / 16.5 / 17.2, 3000 rows (96, 376) 27.7 / 16.0 /
+// 14.1.  The persistent blocks are the fastest at any row count that they fill
+// (N 2048 K 512, 8103 rows 132.0; N 1024 K 256, 16,000 rows 71.9 against
+// 85.1).
 int gemm_f32_config(const GemmArgs& a) {
   if (a.M >= 16384) return a.N >= 256 ? 0 : 1;
+  const long long n64 = (a.N + 63) / 64, n32 = (a.N + 31) / 32;
+  if ((a.M + 127) / 128 * n64 >= 700) return 1;
+  if (a.K % 32 == 0 && (a.M + 63) / 64 * n32 >= 500) return 3;
   return 2;
 }
 
@@ -603,18 +617,18 @@ hipError_t gemm_f32_ln(const GemmArgs& a, const LnEpi& ln, hipStream_t s) {
 hipError_t gemm_f32(const GemmArgs& a, hipStream_t s) {
   if (a.M <= 0 || a.N <= 0) return hipSuccess;
   if (a.K % 16 != 0 || a.ldx % 4 != 0 || a.ldw % 4 != 0) return hipErrorInvalidValue;
+  if (f32_persist_fits(a) && f32_persist_fills(a)) {
+    switch (a.act) {
+      case ACT_NONE: return f32_persist_go<ACT_NONE>(a, s);
+      case ACT_GELU: return f32_persist_go<ACT_GELU>(a, s);
+      case ACT_RELU: return f32_persist_go<ACT_RELU>(a, s);
+      default: return hipErrorInvalidValue;
+    }
+  }
   switch (gemm_f32_config(a)) {
-    case 0:
-      if (f32_persist_fits(a) && f32_persist_fills(a)) {
-        switch (a.act) {
-          case ACT_NONE: return f32_persist_go<ACT_NONE>(a, s);
-          case ACT_GELU: return f32_persist_go<ACT_GELU>(a, s);
-          case ACT_RELU: return f32_persist_go<ACT_RELU>(a, s);
-          default: return hipErrorInvalidValue;
-        }
-      }
-      return launch_cfg<128, 256, 4, 4, 16>(a, s);
+    case 0: return launch_cfg<128, 256, 4, 4, 16>(a, s);
     case 1: return launch_cfg<128, 64, 4, 2, 16>(a, s);
+    case 3: return launch_cfg<64, 32, 4, 2, 32>(a, s);
     default:
       return a.K % 32 == 0 ? launch_cfg<32, 32, 2, 2, 32>(a, s) : launch_cfg<32, 32, 2, 2, 16>(a, s);
   }

@@ -32,3 +32,30 @@ def test_rows_around_tiles(make_weights, d, rows):
     assert bool((got[rows:] == -7.0).all())
     assert torch.equal(got[:rows].view(torch.int32), want.view(torch.int32))
     c.close()
+
+
+@pytest.mark.parametrize("d,rows", [(64, 15873), (80, 9001), (256, 3969), (256, 5505),
+                                    (256, 16383), (512, 2049), (512, 8104)])
+def test_mid_size_rows(make_weights, d, rows):
+    """Fewer rows than a compress tile's run 128x64, 64x32 or 32x32 blocks by
+    how many of them there are, or persistent blocks that fill the CUs: at
+    rows around those lines the logits equal those of 200-row calls (32x32)."""
+    import torch
+
+    import boa_hip
+    c = boa_hip.Codec(d, 1, 16, rows)
+    c.set_stream(torch.cuda.current_stream().cuda_stream)
+    c.load_weights(make_weights(d, 1))
+    tok = torch.from_numpy(np.random.default_rng(rows).integers(0, 256, rows, dtype=np.uint8)).cuda()
+    c.reset_state(rows)
+    got = torch.full((rows + 300, 256), -7.0, device="cuda")
+    c.forward_chunk(tok, rows, 1, got)
+    want = torch.zeros((rows, 256), device="cuda")
+    for r in range(0, rows, 200):
+        n = min(200, rows - r)
+        c.reset_state(n)
+        c.forward_chunk(tok[r:r + n].contiguous(), n, 1, want[r:r + n])
+    torch.cuda.synchronize()
+    assert bool((got[rows:] == -7.0).all())
+    assert torch.equal(got[:rows].view(torch.int32), want.view(torch.int32))
+    c.close()
