@@ -231,8 +231,11 @@ __device__ __forceinline__ void cdf_row_lowprob(const float* lg, const CdfEpi& c
   }
 }
 
+__device__ __forceinline__ uint32_t q_lower(double c, int k) {
+  return (uint32_t)(c * CDF_SCALE) + (uint32_t)k;
+}
 __device__ __forceinline__ uint32_t q_low(const double* s_cdf, int k) {
-  return (uint32_t)(s_cdf[k] * CDF_SCALE) + (uint32_t)k;
+  return q_lower(s_cdf[k], k);
 }
 __device__ __forceinline__ uint32_t q_high(const double* s_cdf, int k) {
   return k == 255 ? TOTAL : (uint32_t)(s_cdf[k + 1] * CDF_SCALE) + (uint32_t)(k + 1);

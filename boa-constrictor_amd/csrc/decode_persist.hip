@@ -36,27 +36,39 @@ constexpr int PL = 16;  // MFMA rows of the block's tiles: the lane capacity of 
 // ((k / 16) 16 + m) 16 + dperm(k % 16)); W: k-blocked decode weights in
 // global memory with capacity ldw.  Lane (i, g) feeds W row n0 + i and lane
 // i's float4 g of every 16-k block, four MFMAs per block in k order -- the
-// arrangement of dec_mainloop.
+// arrangement of dec_mainloop.  The weights do not depend on the step: a wave
+// loads its tile's (pd_load) phases ahead of the MFMAs (pd_mac), and the
+// barriers between wait for LDS only.
 template <int KB>
-__device__ __forceinline__ floatx4 pd_tile(const float* A, const float* __restrict__ W, int ldw,
-                                           int n0, int i, int g) {
-  const float4* w4 = reinterpret_cast<const float4*>(W) + (size_t)(n0 + i) * 4 + g;
-  const size_t wq = (size_t)ldw * 4;
-  constexpr int CH = KB < 8 ? KB : 8;  // weight float4s loaded ahead of their MFMAs
+__device__ __forceinline__ void pd_load(float4* wv, const float* __restrict__ W, int ldw, int n0,
+                                        int i, int g) {
+  // uniform base, one 32-bit lane offset for all loads
+  const char* base = reinterpret_cast<const char*>(W) + n0 * 64;
+  const uint32_t off = (uint32_t)(i * 64 + g * 16);
+#pragma unroll
+  for (int q = 0; q < KB; ++q)
+    wv[q] = *reinterpret_cast<const float4*>(base + (size_t)q * ldw * 64 + off);
+}
+
+// Registers that another wave fills: any value, from no instruction (without
+// it they would keep, and spill, the last loop iteration's)
+template <int KB>
+__device__ __forceinline__ void pd_none(float4* wv) {
+#pragma unroll
+  for (int q = 0; q < KB; ++q)
+    asm volatile("" : "=v"(wv[q].x), "=v"(wv[q].y), "=v"(wv[q].z), "=v"(wv[q].w));
+}
+
+template <int KB>
+__device__ __forceinline__ floatx4 pd_mac(const float* A, const float4* wv, int i, int g) {
   floatx4 acc = floatx4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-  for (int q0 = 0; q0 < KB; q0 += CH) {
-    float4 wv[CH];
-#pragma unroll
-    for (int q = 0; q < CH; ++q) wv[q] = w4[(size_t)(q0 + q) * wq];
-#pragma unroll
-    for (int q = 0; q < CH; ++q) {
-      const float4 bv = reinterpret_cast<const float4*>(A + ((q0 + q) * PL + i) * 16)[g];
-      acc = __builtin_amdgcn_mfma_f32_16x16x4f32(wv[q].x, bv.x, acc, 0, 0, 0);
-      acc = __builtin_amdgcn_mfma_f32_16x16x4f32(wv[q].y, bv.y, acc, 0, 0, 0);
-      acc = __builtin_amdgcn_mfma_f32_16x16x4f32(wv[q].z, bv.z, acc, 0, 0, 0);
-      acc = __builtin_amdgcn_mfma_f32_16x16x4f32(wv[q].w, bv.w, acc, 0, 0, 0);
-    }
+  for (int q = 0; q < KB; ++q) {
+    const float4 bv = reinterpret_cast<const float4*>(A + (q * PL + i) * 16)[g];
+    acc = __builtin_amdgcn_mfma_f32_16x16x4f32(wv[q].x, bv.x, acc, 0, 0, 0);
+    acc = __builtin_amdgcn_mfma_f32_16x16x4f32(wv[q].y, bv.y, acc, 0, 0, 0);
+    acc = __builtin_amdgcn_mfma_f32_16x16x4f32(wv[q].z, bv.z, acc, 0, 0, 0);
+    acc = __builtin_amdgcn_mfma_f32_16x16x4f32(wv[q].w, bv.w, acc, 0, 0, 0);
   }
   return acc;
 }
@@ -151,10 +163,22 @@ __device__ __forceinline__ void pd_ln_apply(const float* xs, float* xn, const fl
 // a block's matrix-core chains cost the same for any LP, while its VALU
 // phases (the scan's 16 exponentials per channel, GELU, the CDF) scale with
 // LP.  Fewer lanes per block spread those phases over more CUs.
+//
+// What bounds it: a serial chain.  A step is 30 phases between barriers, in
+// which an MFMA chain of K / 4 takes 42 cycles per MFMA (256 features at once:
+// 2048 cycles a SIMD), and the elementwise phases their instruction latency.
+// So everything that does not depend on the phase before is out of the chain:
+// weights and recurrent states are loaded phases ahead into registers, MFMA
+// outputs of LP < 16 lanes are spread over the wave before GELU and the conv
+// step, the coder's division runs under out_proj, and the symbol search stays
+// in the registers of the CDF (µs per step at 2 layers: 1 to 512 lanes 34.7 ->
+// 25.5, 1024 lanes 42.8 -> 27.9, 4096 lanes 58.7 -> 40.4; 2 lanes per block
+// gave 25.0 up to 300 lanes, 26.5 at 512).
 template <int NB, int RB, int LP>
 __global__ __launch_bounds__(1024) void dec_persist_kernel(PersistArgs a) {
   static_assert(LP == 4 || LP == 8 || LP == 16, "lanes per block");
   constexpr int LSH = LP == 4 ? 2 : LP == 8 ? 3 : 4;
+  constexpr int VPL = LP / 4;  // values per thread of PD_SPREAD
   constexpr int d = NB * 16, DI = 2 * d, NBI = 2 * NB, NBF = 4 * NB, DS = 16;
   constexpr int NBX = (RB + 2 * DS + 15) / 16;  // 16-blocks of the x_proj row
   constexpr int RW = NBX * 16 + 1;              // LDS row stride of the x_proj rows
@@ -167,7 +191,6 @@ __global__ __launch_bounds__(1024) void dec_persist_kernel(PersistArgs a) {
   __shared__ __align__(16) float os[NB * 256];   // out_proj / head1 output
   __shared__ __align__(16) float hid[NBF * 256]; // FF1 output
   __shared__ __align__(16) float lg[PL * 256];   // logits, row-major
-  __shared__ double s_cdf[PL][260];
   __shared__ float stats[2 * PL];
   __shared__ int tok_s[PL];
   // per-channel parameters of every layer and the head biases, staged once
@@ -193,6 +216,7 @@ __global__ __launch_bounds__(1024) void dec_persist_kernel(PersistArgs a) {
   const uint32_t* pin = nullptr;
   int32_t pn = 0;
   uint32_t nw = 0;
+  uint32_t target0 = 0;
   if (coder_lane && l == 0) {
     pin = a.payload + a.offsets[mh];
     pn = a.sizes[mh];
@@ -218,132 +242,227 @@ __global__ __launch_bounds__(1024) void dec_persist_kernel(PersistArgs a) {
   stage(hb2, a.hb2, 256);
   __syncthreads();
 
+  static_assert(2 * NBI == 16 && NBF == 16, "one in_proj and FF1 tile per wave");
+  // Weight tiles in flight: every wave's tile of in_proj, FF1, then the next
+  // layer's in_proj or head2; and, of waves 0 .. 3, head1's.
+  float4 wa[NB], wh[NB];
+  pd_load<NB>(wa, a.layer[0].w_in, 2 * DI, (tid0 >> 6) * 16, tid0 & 15, (tid0 >> 4) & 3);
+
+  const int wv = __builtin_amdgcn_readfirstlane(tid0 >> 6);
+
   for (int t = 1; t < a.maxlen; ++t) {
-    // the thread index passes through an opaque move each step, so that the
-    // many addresses derived from it are recomputed in the step instead of
-    // being hoisted out of the loop (and spilled)
-    int tid = tid0;
-    asm volatile("" : "+v"(tid));
-    const int wv = tid >> 6, i = tid & 15, g = (tid >> 4) & 3;
-    const int mi = min(m0 + min(i, LP - 1), a.lanes - 1);  // lane of MFMA row i (state index)
-    const bool mi_ok = i < LP && m0 + i < a.lanes;
-#pragma unroll
-    for (int li = 0; li < PERSIST_MAX_LAYERS; ++li) {  // unrolled: constant kernel-argument offsets
-      if (li >= a.L) break;
+    // the thread index passes through an opaque move in each phase (PD_IDX),
+    // so that the many addresses derived from it are recomputed there instead
+    // of being hoisted out of the loop (and spilled)
+#define PD_IDX                  \
+  int tid = tid0;               \
+  asm volatile("" : "+v"(tid)); \
+  [[maybe_unused]] const int i = tid & 15, g = (tid >> 4) & 3
+    {  // x = embedding rows of the current tokens
+      PD_IDX;
+      for (int p = tid; p < NB * 256; p += 1024) {
+        const int q = p >> 8, m = (p >> 4) & 15;
+        xs[p] = a.emb[(size_t)tok_s[m] * d + 16 * q + dperm(p & 15)];
+      }
+    }
+    __syncthreads();
+    // An MFMA tile's 16 features of the block's LP lanes, spread over all
+    // lanes of the wave (through its LDS tile) for the elementwise work on
+    // it: thread (i, g) takes lane m, components e0 .. e0 + VPL - 1 of lane
+    // m's float4 g
+#define PD_SPREAD const int m = i & (LP - 1), e0 = (i >> LSH) * VPL
+#pragma unroll 1
+    for (int li = 0; li < a.L; ++li) {
       const PersistLayer& P = a.layer[li];
       const float* q = prm + li * PSZ;
-      if (li == 0) {  // x = embedding rows of the current tokens
-        for (int p = tid; p < NB * 256; p += 1024) {
-          const int q = p >> 8, m = (p >> 4) & 15;
-          xs[p] = a.emb[(size_t)tok_s[m] * d + 16 * q + dperm(p & 15)];
+      float4 s0[VPL];  // conv state of in_proj's tile
+      float4 wx[NBI];  // x_proj's weights, waves 0 ..
+      float4 wq[NBF];  // out_proj's (waves 8 .. 11) and FF2's (waves 12 .. 15)
+      {
+        PD_IDX;
+        if (wv < NBX)
+          pd_load<NBI>(wx, P.w_x, NBX * 16, wv * 16, i, g);
+        else
+          pd_none<NBI>(wx);
+        if (wv < NBI) {
+          PD_SPREAD;
+#pragma unroll
+          for (int k = 0; k < VPL; ++k)
+            s0[k] = reinterpret_cast<const float4*>(P.conv)[(size_t)(wv * 16 + 4 * (e0 + k) + g) * a.ld_state +
+                                                            min(m0 + m, a.lanes - 1)];
+        } else {
+          pd_none<VPL>(s0);
         }
-        __syncthreads();
+        pd_ln_stats<1, NB>(xs, stats, tid, a.ln_n);
       }
-      pd_ln_stats<1, NB>(xs, stats, tid, a.ln_n);
       __syncthreads();
-      pd_ln_apply<1, NB>(xs, xn, stats, q + O_LN1W, q + O_LN1B, tid, a.ln_n);
+      {
+        PD_IDX;
+        pd_ln_apply<1, NB>(xs, xn, stats, q + O_LN1W, q + O_LN1B, tid, a.ln_n);
+      }
       __syncthreads();
       // in_proj: features < DI run the conv step (state float4 [c][lane]),
       // features >= DI are z
-      for (int tile = wv; tile < 2 * NBI; tile += 16) {
-        const int n0 = tile * 16;
-        float4 s0[4];  // conv state, loaded ahead of the MFMA chain
+      {
+        PD_IDX;
+        const int n0 = wv * 16;
+        const floatx4 acc = pd_mac<NB>(xn, wa, i, g);
+        pd_load<NB>(wa, P.w1, 4 * d, n0, i, g);
         if (n0 < DI) {
+          PD_SPREAD;
+          if (i < LP) *pd_out(cvs, n0, i, g) = make_float4(acc[0], acc[1], acc[2], acc[3]);
+          __builtin_amdgcn_wave_barrier();
+          float* const sp = reinterpret_cast<float*>(pd_out(cvs, n0, m, g)) + e0;
 #pragma unroll
-          for (int e = 0; e < 4; ++e)
-            s0[e] = reinterpret_cast<const float4*>(P.conv)[(size_t)(n0 + 4 * e + g) * a.ld_state + mi];
-        }
-        const floatx4 acc = pd_tile<NB>(xn, P.w_in, 2 * DI, n0, i, g);
-        float v[4];
-#pragma unroll
-        for (int e = 0; e < 4; ++e) v[e] = acc[e] + q[O_BIN + n0 + 4 * e + g];
-        if (n0 < DI) {
-          float cv[4];
-#pragma unroll
-          for (int e = 0; e < 4; ++e) {
-            const int n = n0 + 4 * e + g;
+          for (int k = 0; k < VPL; ++k) {
+            const int n = n0 + 4 * (e0 + k) + g;
+            const float v = sp[k] + q[O_BIN + n];
             const float4 cw = reinterpret_cast<const float4*>(q + O_CONVW)[n];
-            cv[e] = conv_step_value<MATH_BR>(q[O_CONVB + n], s0[e], v[e], cw);
-            if (mi_ok)
-              reinterpret_cast<float4*>(P.conv)[(size_t)n * a.ld_state + mi] =
-                  make_float4(s0[e].y, s0[e].z, s0[e].w, v[e]);
+            const float cv = conv_step_value<MATH_BR>(q[O_CONVB + n], s0[k], v, cw);
+            sp[k] = cv;
+            if (m0 + m < a.lanes)
+              reinterpret_cast<float4*>(P.conv)[(size_t)n * a.ld_state + m0 + m] =
+                  make_float4(s0[k].y, s0[k].z, s0[k].w, v);
           }
-          *pd_out(cvs, n0, i, g) = make_float4(cv[0], cv[1], cv[2], cv[3]);
         } else {
+          float v[4];
+#pragma unroll
+          for (int e = 0; e < 4; ++e) v[e] = acc[e] + q[O_BIN + n0 + 4 * e + g];
           *pd_out(zs, n0 - DI, i, g) = make_float4(v[0], v[1], v[2], v[3]);
         }
       }
+      // scan item it: lane (it / 16) % LP, channel 16 (it / 16 / LP) + it % 16;
+      // the first item's state is loaded here
+      float4* const h4 = reinterpret_cast<float4*>(P.ssm);
+      float4 hv[DS / 4];
+      auto load_h = [&](int it) {
+        const int cl = it & 15, lm = (it >> 4) & (LP - 1), cb = it >> (4 + LSH);
+        const int m = min(m0 + lm, a.lanes - 1);
+#pragma unroll
+        for (int n4 = 0; n4 < DS / 4; ++n4)
+          hv[n4] = h4[((size_t)(cb * (DS / 4) + n4) * a.ld_state + m) * 16 + cl];
+      };
+      auto load_after_scan = [&](int i, int g) {  // out_proj's and FF2's weights
+        if (wv >= 12) {
+          pd_load<NBF>(wq, P.w2, d, (wv - 12) * 16, i, g);
+        } else if (wv >= 8) {
+          pd_load<NBI>(wq, P.w_out, d, (wv - 8) * 16, i, g);
+          pd_none<NBF - NBI>(wq + NBI);
+        } else {
+          pd_none<NBF>(wq);
+        }
+      };
+      if (LP * DI >= 1024 || wv < LP * DI / 64) {
+        PD_IDX;
+        load_h(tid);
+      } else {
+        pd_none<DS / 4>(hv);
+      }
       __syncthreads();
       // x_proj (no bias: + 0 as the step's epilogue)
-      for (int tile = wv; tile < NBX; tile += 16) {
-        const floatx4 acc = pd_tile<NBI>(cvs, P.w_x, NBX * 16, tile * 16, i, g);
+      if (wv < NBX) {
+        PD_IDX;
+        const floatx4 acc = pd_mac<NBI>(cvs, wx, i, g);
 #pragma unroll
-        for (int e = 0; e < 4; ++e) rwn[i * RW + tile * 16 + 4 * e + g] = acc[e] + 0.0f;
+        for (int e = 0; e < 4; ++e) rwn[i * RW + wv * 16 + 4 * e + g] = acc[e] + 0.0f;
       }
       __syncthreads();
-      // scan: item (lane lm, channel c), the operations of dec_scan_kernel
+      // scan: the operations of dec_scan_kernel
+      if (LP * DI >= 1024 || wv < LP * DI / 64) {
+        PD_IDX;
 #pragma unroll 1
-      for (int it = tid; it < LP * DI; it += 1024) {
-        const int cl = it & 15, lm = (it >> 4) & (LP - 1), cb = it >> (4 + LSH);
-        const int c = cb * 16 + cl;
-        const int m = min(m0 + lm, a.lanes - 1);
-        float4* h4 = reinterpret_cast<float4*>(P.ssm);
-        const float4* na4 = reinterpret_cast<const float4*>(q + O_NAQ);
-        const float4* w4 = reinterpret_cast<const float4*>(q + O_WDTQ);
-        ScanCtx<DS, RB> sc;
+        for (int it = tid; it < LP * DI; it += 1024) {
+          const int cl = it & 15, lm = (it >> 4) & (LP - 1), cb = it >> (4 + LSH);
+          const int c = cb * 16 + cl;
+          const int m = min(m0 + lm, a.lanes - 1);
+          const float4* na4 = reinterpret_cast<const float4*>(q + O_NAQ);
+          const float4* w4 = reinterpret_cast<const float4*>(q + O_WDTQ);
+          ScanCtx<DS, RB> sc;
 #pragma unroll
-        for (int n4 = 0; n4 < DS / 4; ++n4) {
-          const float4 hv = h4[((size_t)(cb * (DS / 4) + n4) * a.ld_state + m) * 16 + cl];
-          sc.h[4 * n4] = hv.x; sc.h[4 * n4 + 1] = hv.y; sc.h[4 * n4 + 2] = hv.z; sc.h[4 * n4 + 3] = hv.w;
-          const float4 av = na4[(cb * (DS / 4) + n4) * 16 + cl];
-          sc.na[4 * n4] = av.x; sc.na[4 * n4 + 1] = av.y; sc.na[4 * n4 + 2] = av.z; sc.na[4 * n4 + 3] = av.w;
-        }
+          for (int n4 = 0; n4 < DS / 4; ++n4) {
+            sc.h[4 * n4] = hv[n4].x; sc.h[4 * n4 + 1] = hv[n4].y;
+            sc.h[4 * n4 + 2] = hv[n4].z; sc.h[4 * n4 + 3] = hv[n4].w;
+            const float4 av = na4[(cb * (DS / 4) + n4) * 16 + cl];
+            sc.na[4 * n4] = av.x; sc.na[4 * n4 + 1] = av.y; sc.na[4 * n4 + 2] = av.z; sc.na[4 * n4 + 3] = av.w;
+          }
 #pragma unroll
-        for (int j4 = 0; j4 < RB / 4; ++j4) {
-          const float4 wd = w4[(cb * (RB / 4) + j4) * 16 + cl];
-          sc.wdt[4 * j4] = wd.x; sc.wdt[4 * j4 + 1] = wd.y; sc.wdt[4 * j4 + 2] = wd.z; sc.wdt[4 * j4 + 3] = wd.w;
-        }
-        sc.bdt = q[O_BDT + c];
-        sc.dd = q[O_DD + c];
-        const float* row = rwn + lm * RW;
-        const int cp = ((c >> 4) * PL + lm) * 16 + dperm(c & 15);
-        ys[cp] = scan_token<DS, RB, MATH_BR>(sc, row, row + RB, a.r, cvs[cp], zs[cp]);
-        if (m0 + lm < a.lanes) {
+          for (int j4 = 0; j4 < RB / 4; ++j4) {
+            const float4 wd = w4[(cb * (RB / 4) + j4) * 16 + cl];
+            sc.wdt[4 * j4] = wd.x; sc.wdt[4 * j4 + 1] = wd.y; sc.wdt[4 * j4 + 2] = wd.z; sc.wdt[4 * j4 + 3] = wd.w;
+          }
+          sc.bdt = q[O_BDT + c];
+          sc.dd = q[O_DD + c];
+          const float* row = rwn + lm * RW;
+          const int cp = ((c >> 4) * PL + lm) * 16 + dperm(c & 15);
+          ys[cp] = scan_token<DS, RB, MATH_BR>(sc, row, row + RB, a.r, cvs[cp], zs[cp]);
+          if (m0 + lm < a.lanes) {
 #pragma unroll
-          for (int n4 = 0; n4 < DS / 4; ++n4)
-            h4[((size_t)(cb * (DS / 4) + n4) * a.ld_state + m) * 16 + cl] =
-                make_float4(sc.h[4 * n4], sc.h[4 * n4 + 1], sc.h[4 * n4 + 2], sc.h[4 * n4 + 3]);
+            for (int n4 = 0; n4 < DS / 4; ++n4)
+              h4[((size_t)(cb * (DS / 4) + n4) * a.ld_state + m) * 16 + cl] =
+                  make_float4(sc.h[4 * n4], sc.h[4 * n4 + 1], sc.h[4 * n4 + 2], sc.h[4 * n4 + 3]);
+          }
+          if (LP * DI > 1024 && it + 1024 < LP * DI) load_h(it + 1024);
         }
+        if (LP * DI >= 1024)
+          load_after_scan(i, g);
+        else
+          pd_none<NBF>(wq);
+      } else {
+        PD_IDX;
+        load_after_scan(i, g);  // these waves have no scan items
       }
       __syncthreads();
+      // (the coder's division, on waves that have nothing else here)
+      if (coder_lane && l == 0 && li == 0) target0 = dec_target(st);
       // out_proj + bias
-      for (int tile = wv; tile < NB; tile += 16) {
-        const int n0 = tile * 16;
-        const floatx4 acc = pd_tile<NBI>(ys, P.w_out, d, n0, i, g);
+      if (wv >= 8 && wv < 12) {
+        PD_IDX;
+        const int n0 = (wv - 8) * 16;
+        const floatx4 acc = pd_mac<NBI>(ys, wq, i, g);
         float v[4];
 #pragma unroll
         for (int e = 0; e < 4; ++e) v[e] = acc[e] + q[O_BOUT + n0 + 4 * e + g];
         *pd_out(os, n0, i, g) = make_float4(v[0], v[1], v[2], v[3]);
       }
       __syncthreads();
-      pd_ln_stats<2, NB>(os, stats, tid, a.ln_n);
+      {
+        PD_IDX;
+        pd_ln_stats<2, NB>(os, stats, tid, a.ln_n);
+      }
       __syncthreads();
-      pd_ln_apply<2, NB>(os, xn, stats, q + O_LN2W, q + O_LN2B, tid, a.ln_n);
+      {
+        PD_IDX;
+        pd_ln_apply<2, NB>(os, xn, stats, q + O_LN2W, q + O_LN2B, tid, a.ln_n);
+      }
       __syncthreads();
       // FF1 + bias + GELU
-      for (int tile = wv; tile < NBF; tile += 16) {
-        const int n0 = tile * 16;
-        const floatx4 acc = pd_tile<NB>(xn, P.w1, 4 * d, n0, i, g);
-        float v[4];
+      {
+        PD_IDX;
+        const int n0 = wv * 16;
+        const floatx4 acc = pd_mac<NB>(xn, wa, i, g);
+        const bool more = li + 1 < a.L;
+        pd_load<NB>(wa, more ? a.layer[li + 1 < PERSIST_MAX_LAYERS ? li + 1 : li].w_in : a.hw2, 256,
+                    n0, i, g);
+        PD_SPREAD;
+        if (i < LP) *pd_out(hid, n0, i, g) = make_float4(acc[0], acc[1], acc[2], acc[3]);
+        __builtin_amdgcn_wave_barrier();
+        float* const sp = reinterpret_cast<float*>(pd_out(hid, n0, m, g)) + e0;
 #pragma unroll
-        for (int e = 0; e < 4; ++e) v[e] = gelu<MATH_BR>(acc[e] + q[O_B1 + n0 + 4 * e + g]);
-        *pd_out(hid, n0, i, g) = make_float4(v[0], v[1], v[2], v[3]);
+        for (int k = 0; k < VPL; ++k) {
+          const float v = gelu<MATH_BR>(sp[k] + q[O_B1 + n0 + 4 * (e0 + k) + g]);
+          sp[k] = v;
+        }
+        if (!more && wv < NB)
+          pd_load<NB>(wh, a.hw1, d, n0, i, g);
+        else
+          pd_none<NB>(wh);
       }
       __syncthreads();
       // FF2 + bias + residual (each float4 of x read and written by one lane)
-      for (int tile = wv; tile < NB; tile += 16) {
-        const int n0 = tile * 16;
-        const floatx4 acc = pd_tile<NBF>(hid, P.w2, d, n0, i, g);
+      if (wv >= 12) {
+        PD_IDX;
+        const int n0 = (wv - 12) * 16;
+        const floatx4 acc = pd_mac<NBF>(hid, wq, i, g);
         float4* xp = pd_out(xs, n0, i, g);
         const float4 rv = *xp;
         float v[4];
@@ -354,9 +473,10 @@ __global__ __launch_bounds__(1024) void dec_persist_kernel(PersistArgs a) {
       __syncthreads();
     }
     // head1 + bias + ReLU
-    for (int tile = wv; tile < NB; tile += 16) {
-      const int n0 = tile * 16;
-      const floatx4 acc = pd_tile<NB>(xs, a.hw1, d, n0, i, g);
+    if (wv < NB) {
+      PD_IDX;
+      const int n0 = wv * 16;
+      const floatx4 acc = pd_mac<NB>(xs, wh, i, g);
       float v[4];
 #pragma unroll
       for (int e = 0; e < 4; ++e) v[e] = fmaxf(0.0f, acc[e] + hb1[n0 + 4 * e + g]);
@@ -365,47 +485,48 @@ __global__ __launch_bounds__(1024) void dec_persist_kernel(PersistArgs a) {
     __syncthreads();
     // head2, row-major (unpermuted weights: component e is feature n0 + 4 g + e),
     // without b2 (the CDF adds it)
-    for (int tile = wv; tile < 16; tile += 16) {
-      const int n0 = tile * 16;
-      const floatx4 acc = pd_tile<NB>(os, a.hw2, 256, n0, i, g);
+    {
+      PD_IDX;
+      const int n0 = wv * 16;
+      const floatx4 acc = pd_mac<NB>(os, wa, i, g);
+      pd_load<NB>(wa, a.layer[0].w_in, 2 * DI, n0, i, g);
       *reinterpret_cast<float4*>(lg + i * 256 + n0 + 4 * g) =
           make_float4(acc[0] + 0.0f, acc[1] + 0.0f, acc[2] + 0.0f, acc[3] + 0.0f);
     }
     __syncthreads();
-    // CDF of each lane's row on its half-wave
+    // CDF of each lane's row on its half-wave (lane l: symbols 8 l .. 8 l + 7),
+    // symbol search (the lowest symbol whose range holds the target: ballot,
+    // first set bit, first of the lane's eight) and the coder advance
     if (half < LP) {
       double r[8];
       cdf_halfwave_regs(lg + half * 256, hb2, a.inv_t, l, r);
+      if (coder_lane && t < len_h) {  // uniform over the half-wave
+        const uint32_t target = __shfl(target0, 0, 32);
+        uint32_t lo[9];
 #pragma unroll
-      for (int k = 0; k < 8; ++k) s_cdf[half][8 * l + k] = r[k];
-      if (l == 31) s_cdf[half][256] = 1.0;
-    }
-    __syncthreads();
-    // symbol search (8 rounds of 32 candidates, ballot + first set bit) and
-    // the coder advance, as decode_step_kernel
-    if (coder_lane && t < len_h) {  // uniform over the half-wave
-      const uint32_t target = __shfl(l == 0 ? dec_target(st) : 0u, 0, 32);
-      const double* sc = s_cdf[half];
-      int sym = 0;
-      uint32_t low_s = 0, high_s = 0;
-      const int shift = tid0 & 32;
-      for (int round = 0; round < 8; ++round) {
-        const int k = round * 32 + l;
-        const uint32_t lo = q_low(sc, k), hi = q_high(sc, k);
-        const bool match = target >= lo && target < hi;
-        const uint32_t mask = (uint32_t)(__ballot(match) >> shift);
-        if (mask != 0u) {
-          const int winner = __ffs(mask) - 1;
-          sym = __shfl(k, winner, 32);
-          low_s = __shfl(lo, winner, 32);
-          high_s = __shfl(hi, winner, 32);
-          break;
+        for (int k = 0; k < 8; ++k) lo[k] = q_lower(r[k], 8 * l + k);
+        const uint32_t next = __shfl_down(lo[0], 1, 32);
+        lo[8] = l == 31 ? TOTAL : next;
+        int sym = -1;
+        uint32_t low = 0, high = 0;
+#pragma unroll
+        for (int k = 7; k >= 0; --k)
+          if (target >= lo[k] && target < lo[k + 1]) {
+            sym = 8 * l + k;
+            low = lo[k];
+            high = lo[k + 1];
+          }
+        const uint32_t mask = (uint32_t)(__ballot(sym >= 0) >> (tid0 & 32));
+        const int winner = mask != 0u ? __ffs(mask) - 1 : 0;
+        sym = __shfl(sym, winner, 32);
+        low = __shfl(low, winner, 32);
+        high = __shfl(high, winner, 32);
+        if (mask == 0u) sym = 0, low = 0, high = 0;
+        if (l == 0) {
+          dec_advance_ahead(st, low, high, pin, pn, nw);
+          a.out[(size_t)mh * a.out_stride + t] = (uint8_t)sym;
+          tok_s[half] = sym;
         }
-      }
-      if (l == 0) {
-        dec_advance_ahead(st, low_s, high_s, pin, pn, nw);
-        a.out[(size_t)mh * a.out_stride + t] = (uint8_t)sym;
-        tok_s[half] = sym;
       }
     }
     __syncthreads();
