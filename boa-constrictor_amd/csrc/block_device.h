@@ -317,19 +317,19 @@ __device__ __forceinline__ float scan_token_any(float (&h)[DS], const P& p, cons
   const float y = scan_states<DS, M, false>(h, p, row, dt, u) + p.dd() * u;
   return y * (z * (M == MATH_HW ? sigmoid<M>(z) : sigmoid_any<M>(z)));
 }
+// One token of a decode step, in the general form: the step's scan waits for
+// its state, and a second form of the token beside it cost 0.3 % of a step
+// (decompress of 4096 lanes, d_model 256: 145.9 -> 146.5 ms).
 template <int DS, int RB, int M, class P>
 __device__ __forceinline__ float scan_token_p(float (&h)[DS], const P& p, const float* dt_in,
                                               const float* bc, int r, float u, float z) {
   const RowFloats<DS> row{dt_in, bc};
   const float x = scan_x<RB>(p, row, r);
-  if (M != MATH_HW && scan_ordinary(p, x, z))
-    return scan_token_ordinary<DS, M, P::CORE>(h, p, row, x, u, z);
   return scan_token_any<DS, M>(h, p, row, x, u, z);
 }
 template <int DS, int RB>
 struct ScanRegs {
   const ScanCtx<DS, RB>& c;
-  static constexpr bool CORE = true;
   __device__ __forceinline__ float xmax() const { return c.xmax; }
   __device__ __forceinline__ float wdt(int j) const { return c.wdt[j]; }
   __device__ __forceinline__ float na(int n) const { return c.na[n]; }
@@ -346,8 +346,6 @@ template <int DS, int RB>
 struct ScanLds {
   const float* p;
   int cl;
-  static constexpr bool CORE = false;  // no per-channel limit kept: exp2_neg clamps
-  __device__ __forceinline__ float xmax() const { return ORDINARY; }
   __device__ __forceinline__ float na(int n) const { return p[((n >> 2) * 16 + cl) * 4 + (n & 3)]; }
   __device__ __forceinline__ float wdt(int j) const {
     return p[DS * 16 + ((j >> 2) * 16 + cl) * 4 + (j & 3)];
@@ -366,6 +364,8 @@ __device__ __forceinline__ const float4* scan_lds_src(const LayerW& Lw, const fl
   const int j = k - (DS + RB) * 4;  // 0-3 b_dt, 4-7 D
   return reinterpret_cast<const float4*>((j < 4 ? Lw.b_dt : Lw.dd) + 16 * c16) + (j & 3);
 }
+// One decode step of a channel whose ScanCtx the caller filled (xmax is not
+// needed)
 template <int DS, int RB, int M = MATH_BF>
 __device__ __forceinline__ float scan_token(ScanCtx<DS, RB>& sc, const float* dt_in,
                                             const float* bc, int r, float u, float z) {

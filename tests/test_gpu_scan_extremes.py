@@ -63,3 +63,31 @@ def test_scan_limits_match_the_oracle(oracle, tmp_path, d):
             assert np.array_equal(step.cpu().numpy().view(np.uint32),
                                   want[:lanes, t].view(np.uint32)), f"{lanes} lanes, step {t}"
         c.close()
+
+
+@pytest.mark.parametrize("d,lanes", [(64, 5), (64, 2100), (256, 2100)])
+def test_decode_limits_match_the_oracle(oracle, tmp_path, d, lanes):
+    """The persistent decode (d_model 64) and the step's separate scan (above
+    2048 lanes): containers of such weights are the oracle's, decode to the
+    same bytes, and the steps' logits are the chunk forward's."""
+    import torch
+
+    import boa_hip
+    w = tmp_path / "w.bin"
+    _extreme_weights(w, d, 16)
+    T = 9
+    tok = np.random.default_rng(lanes).integers(0, 256, size=(lanes, T), dtype=np.uint8)
+    c = boa_hip.Codec(d, 1, 16, lanes)
+    c.set_stream(torch.cuda.current_stream().cuda_stream)
+    c.load_weights(w)
+    want = oracle.Model(w, d, 1, 16).new_state(lanes).forward_chunk(tok)
+    c.reset_state(lanes)
+    step = torch.zeros((lanes, 256), device="cuda")
+    for t in range(T):
+        c.step_batch(torch.from_numpy(tok[:, t].copy()).cuda(), lanes, step)
+        torch.cuda.synchronize()
+        assert np.array_equal(step.cpu().numpy().view(np.uint32), want[:, t].view(np.uint32))
+    blob = c.compress(tok.tobytes(), chunk_size=T)
+    assert blob == oracle.Model(w, d, 1).compress(tok.tobytes(), chunk_size=T)
+    assert c.decompress(blob) == tok.tobytes()
+    c.close()
