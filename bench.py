@@ -38,8 +38,9 @@ METRIC = ("compress & decompress input MB/s at d256×8L, 1000 chunks; "
           "compression ratio")
 PEAK_TFLOPS = {"fp32": 157.3, "bf16": 2500.0}  # MI355X dense matrix peaks
 PEAK_HBM_GBS = 8000.0     # MI355X HBM3E peak
-GEMM_KERNEL = {"fp32": "boa::gemm_f32_kernel<128, 256, 4, 4, 16, 0|1|2>",
-               "bf16": "boa::gemm_bf16_kernel<256, 256, 4, 4, 64, 1|2, 0|1|2>"}
+GEMM_KERNEL = {"fp32": "boa::gemm_f32_persist_kernel<0|1|2>, "
+                       "gemm_f32_kernel<128, 256, 4, 4, 16, 0|4|5>",
+               "bf16": "boa::gemm_bf16_persist_kernel<0|1|2, 0|1>, ffn_bf16_rows_kernel<1|3>"}
 TRAFFIC_FILE = os.path.join(ROOT, "profiles", "gemm_f32_c2_traffic.json")
 DEC_TRAFFIC_FILE = os.path.join(ROOT, "profiles", "dec_ln_gemm_c2_traffic.json")
 
@@ -201,10 +202,11 @@ def decode_coder_profile(codec, torch, data: bytes, chunk: int, n_chunks: int, s
 # Compiled VALU instructions per element (token x channel) of the compress
 # scan's token loop (scan_chunk_sload_kernel, the large-grid form), counted
 # from this build's gfx950 assembly (hipcc --cuda-device-only -S of mamba.hip;
-# instructions between the loop header and its back branch, one token per
-# iteration): fp32 d_state 16 (the reference's rounding, software exp2) and
-# bf16 (hardware exp; the fused update at d_state 16).
-SCAN_VALU_PER_ELEMENT = {("fp32", 16): 409, ("fp32", 32): 713, ("bf16", 16): 134, ("bf16", 32): 323}
+# instructions between the loop header and its back branch, per token; in fp32
+# the path of ordinary tokens): fp32 d_state 16 (the reference's rounding,
+# software exp2) and bf16 (hardware exp; the fused update at d_state 16, two
+# tokens per iteration).
+SCAN_VALU_PER_ELEMENT = {("fp32", 16): 359, ("fp32", 32): 646, ("bf16", 16): 114, ("bf16", 32): 305}
 # MI355X's published fp32 vector peak, 157.3 TFLOP/s, as wave64 FMA
 # instructions per second (64 lanes x 2 FLOP): 1,228.8 G/s
 VALU_ISSUE_PEAK = 157.3e12 / 128
