@@ -508,13 +508,33 @@ static bool f32_persist_fits(const GemmArgs& a) {
          a.X != a.C;
 }
 
-// Whether the tiles fill the CUs in whole rounds (one block per CU; the 32
-// blocks of an XCD share its m blocks): at 70 % of 3 rounds (17,000 x 2048)
-// the 128 x 256 blocks, finer and two per CU, were 11 % faster, at 50 % 24 %.
-static bool f32_persist_fills(const GemmArgs& a) {
-  const long long mb = (a.M + 255) / 256, nb = a.N / 256;
+// Blocks of bm x bn that the fullest of the 256 CUs gets (they are dispatched
+// round-robin).  The MFMAs of a CU's blocks run one after another however many
+// are resident, so a launch takes about that number times a block's time; a
+// block too many for the CUs costs a whole one.
+static long long cu_blocks(const GemmArgs& a, int bm, int bn) {
+  return (((long long)a.M + bm - 1) / bm * ((a.N + bn - 1) / bn) + 255) / 256;
+}
+
+// Whether the persistent blocks beat the others.  `rounds`: tiles of the
+// busiest CU (the 32 blocks of an XCD share its m blocks).  Below 16,384 rows
+// the alternatives are fine-grained, and the tiles have to fill their rounds:
+// N 2048 K 512 at 7177 rows (0.91 of a round) 132.5 us against 165.2, N 1024 K
+// 256 at 14,441 rows (0.89) 72.6 against 86.1, at 9604 (0.59) 70.4 against
+// 57.0.  From there on against two 128 x 256 blocks a tile, which take 1 /
+// 0.91 of a tile's time; with K below 256 (the output is most of it) 1 / 0.88,
+// with GELU, whose VALU work two resident blocks overlap in part, 1 / 0.96.
+// 2700 points of 16,384 to 800,000 rows, 14 shapes: never more than 4.5 %
+// slower than the 128 x 256 blocks (GELU, K 64), 5.2 % faster in the mean;
+// with one line for all at 0.85 of whole rounds up to 11 % slower (GELU, K 64
+// at 283,705 rows 181.8 us against 163.9; K 512 N 2048 at 35,584 rows 678
+// against 643).
+static bool f32_persist_pays(const GemmArgs& a) {
+  const long long mb = ((long long)a.M + 255) / 256, nb = a.N / 256;
   const long long rounds = ((mb + 7) / 8 * nb + 31) / 32;
-  return 100 * mb * nb >= 85 * 256 * rounds;
+  if (a.M < 16384) return 100 * mb * nb >= 85 * 256 * rounds;
+  const int cost = a.act == ACT_GELU ? 96 : a.K < 256 ? 88 : 91;
+  return 2 * rounds * cost <= 100 * cu_blocks(a, 128, 256);
 }
 
 template <int ACT>
@@ -549,30 +569,32 @@ static hipError_t launch_cfg(const GemmArgs& a, hipStream_t s, int swizzle = 1) 
 }
 
 // Tile choice only changes the schedule, never the numerics (see above).
-// Large M (a compress tile), N >= 256: persistent 256x256 blocks where the
-// shape fits them (TFLOP/s at 1.6 M rows, against 128x256 blocks of 16 waves:
-// K 256 N 1024 113.5 -> 126.6, with GELU at 400,000 rows 98.6 -> 105.9), the
-// 128x256 blocks otherwise (the LayerNorm epilogues and FF2's residual, 256
-// wide: equal to 2 % at whole rounds of the CUs, slower between, and their
-// epilogues overlap the other resident block's MFMAs); 128x64 with 8 waves for
-// the narrow x_proj.
-// Fewer rows (a forward call of some thousand tokens): 128x64 blocks from
-// about three rounds of the CUs (700 blocks) on, 64x32 blocks of eight waves
-// from two rounds (500) on, else 32x32 with four waves, whose finer tiles fill
-// more CUs.  µs of 128x64 / 64x32 / 32x32 at 8103 rows: N 1024 K 256 46.3 /
-// 49.3 / 51.6, N 256 K 512 29.7 / 27.8 / 32.5, N 256 K 1024 53.4 / 48.7 /
-// 60.0, N 2048 K 512 153.9 / 179.4 / 197.4; beside the lines, N 1024 K 256:
-// 6000 rows (752 and 3008 blocks) 37.3 / 38.6 / 39.5, 4000 rows (512, 2016)
-// 27.8 / 27.1 / 28.6, 1000 rows (128, 512) 16.5 / 10.1 / 10.2; N 256 K 512:
-// 4000 rows (128, 504) 27.8 / 16.5 / 17.2, 3000 rows (96, 376) 27.7 / 16.0 /
-// 14.1.  The persistent blocks are the fastest at any row count that they fill
-// (N 2048 K 512, 8103 rows 132.0; N 1024 K 256, 16,000 rows 71.9 against
-// 85.1).
+// Large M (a compress tile), N >= 256: persistent 256x256 blocks where they
+// pay (TFLOP/s at 1.6 M rows, against 128x256 blocks of 16 waves: K 256 N 1024
+// 113.5 -> 126.6, with GELU at 400,000 rows 98.6 -> 105.9), the 128x256 blocks
+// otherwise (the LayerNorm epilogues and FF2's residual, 256 wide: equal to
+// 2 % at whole rounds of the CUs, slower between, and their epilogues overlap
+// the other resident block's MFMAs); 128x64 with 8 waves for the narrow x_proj.
+// Fewer rows (a forward call of some thousand tokens): 32x32 blocks with four
+// waves, unless the fullest CU gets no more work in larger ones, whose MFMAs
+// wait for fewer operands: 128x64 blocks hold eight times the work and are 10
+// to 17 % cheaper for it from K 256 on, so they have to come to less than 1/7 of
+// the number; 64x32 blocks of eight waves twice, 2 to 5 % cheaper from K 512
+// on (below they gain and lose 4 %), so they have to come to half of it.  One
+// of either on a CU exposes its latency (N 256 K 512, 3000 rows: 27.7 us of
+// 128x64, 14.1 of 32x32).  us of 128x64 / 64x32 / 32x32 (blocks on the fullest
+// CU): N 1024 K 256 at 8064 rows 46.7 / 50.5 / 50.8 (4, 16, 32), at 6387 46.1 /
+// 42.0 / 41.6 (4, 13, 25), at 1178 16.4 / 12.8 / 11.4 (2, 3, 5); N 256 K 1024
+// at 8064 rows 51.9 / 49.6 / 53.0 (1, 4, 8), at 4248 50.3 / 38.1 / 34.0 (1, 3,
+// 5); N 2048 K 512 at 10,180 rows 192.8 / 222.4 / 231.5 (10, 40, 80).  2800
+// points of 64 to 16,383 rows, 30 shapes: at most 1.5 % slower than 32x32, up
+// to 18 % faster.
 int gemm_f32_config(const GemmArgs& a) {
   if (a.M >= 16384) return a.N >= 256 ? 0 : 1;
-  const long long n64 = (a.N + 63) / 64, n32 = (a.N + 31) / 32;
-  if ((a.M + 127) / 128 * n64 >= 700) return 1;
-  if (a.K % 32 == 0 && (a.M + 63) / 64 * n32 >= 500) return 3;
+  const long long n128 = cu_blocks(a, 128, 64), n64 = cu_blocks(a, 64, 32),
+                  n32 = cu_blocks(a, 32, 32);
+  if (a.K >= 256 && n128 >= 2 && 7 * n128 < n32) return 1;
+  if (a.K >= 512 && a.K % 32 == 0 && n64 >= 2 && 2 * n64 == n32) return 3;
   return 2;
 }
 
@@ -617,7 +639,7 @@ hipError_t gemm_f32_ln(const GemmArgs& a, const LnEpi& ln, hipStream_t s) {
 hipError_t gemm_f32(const GemmArgs& a, hipStream_t s) {
   if (a.M <= 0 || a.N <= 0) return hipSuccess;
   if (a.K % 16 != 0 || a.ldx % 4 != 0 || a.ldw % 4 != 0) return hipErrorInvalidValue;
-  if (f32_persist_fits(a) && f32_persist_fills(a)) {
+  if (f32_persist_fits(a) && f32_persist_pays(a)) {
     switch (a.act) {
       case ACT_NONE: return f32_persist_go<ACT_NONE>(a, s);
       case ACT_GELU: return f32_persist_go<ACT_GELU>(a, s);

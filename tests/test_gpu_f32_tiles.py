@@ -1,9 +1,9 @@
 """fp32 compress GEMM tiles: from 16,384 rows on the plain GEMMs of 256-wide
 outputs run in 256-row persistent blocks, whose last tile starts early when
-the rows are no multiple of 256, where those tiles fill the CUs.  The row
-counts here are whole rounds of the CUs with 0, 1 and 255 rows over a tile.  The logits of every
-row equal those of short calls (other kernels), and the rows past the last
-one stay untouched."""
+the rows are no multiple of 256, where those tiles pay.  The row counts here
+are whole rounds of the CUs with 0, 1 and 255 rows over a tile, and 0.6 and 0.8
+of a round.  The logits of every row equal those of short calls (other
+kernels), and the rows past the last one stay untouched."""
 import numpy as np
 import pytest
 
@@ -11,7 +11,8 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("d,rows", [(64, 65281), (64, 65535), (256, 16384), (256, 65281),
-                                    (256, 65535), (512, 65535)])
+                                    (256, 65535), (512, 65535), (64, 40001),
+                                    (256, 40961)])
 def test_rows_around_tiles(make_weights, d, rows):
     import torch
 
@@ -38,7 +39,7 @@ def test_rows_around_tiles(make_weights, d, rows):
                                     (256, 16383), (512, 2049), (512, 8104)])
 def test_mid_size_rows(make_weights, d, rows):
     """Fewer rows than a compress tile's run 128x64, 64x32 or 32x32 blocks by
-    how many of them there are, or persistent blocks that fill the CUs: at
+    what they leave the fullest CU, or persistent blocks that fill the CUs: at
     rows around those lines the logits equal those of 200-row calls (32x32)."""
     import torch
 
