@@ -277,7 +277,8 @@ Dims make_dims(const boa_config& cfg) {
   D.di = 2 * D.d;
   D.r = (cfg.d_model + 15) / 16;
   D.ds = cfg.d_state;
-  D.R = D.r + 2 * D.ds;
+  D.rs = cfg.precision == 1 ? (int)round_up(D.r, 2) : D.r;
+  D.R = D.rs + 2 * D.ds;
   D.ld_in = (int)round_up(2 * D.di, 256);
   D.ld_x = (int)round_up(D.R, 256);
   D.ld_out = (int)round_up(D.d, 256);
@@ -288,10 +289,14 @@ Dims make_dims(const boa_config& cfg) {
   return D;
 }
 
+// floats that a row of x_proj's output takes in the activation buffers (in bf16
+// the R elements fill half of them)
+int64_t delta_floats(const Dims& D) { return D.r + 2 * D.ds; }
+
 // compress activation bytes per row: x, xn, xz, conv, delta, y, hidden
 // (floats) and the two (low, prob) buffers
 int64_t row_bytes(const Dims& D) {
-  return 4 * (int64_t)(D.d + D.d + 2 * D.di + D.di + D.R + D.di + 4 * D.d) + 16;
+  return 4 * (D.d + D.d + 2 * D.di + D.di + delta_floats(D) + D.di + 4 * D.d) + 16;
 }
 
 int64_t pitch_words_for(int64_t chunk) { return (chunk * 10 + 4096 + 3) / 4; }
@@ -304,7 +309,7 @@ int ensure_rows(boa_ctx* c, int64_t rows) {
   c->rows_cap = 0;
   size_t r = (size_t)rows;
   if (dalloc(&c->x, r * D.d) || dalloc(&c->xn, r * D.d) || dalloc(&c->xz, r * 2 * D.di) ||
-      dalloc(&c->cv, r * D.di) || dalloc(&c->delta, r * D.R) || dalloc(&c->y, r * D.di) ||
+      dalloc(&c->cv, r * D.di) || dalloc(&c->delta, r * delta_floats(D)) || dalloc(&c->y, r * D.di) ||
       dalloc(&c->hid, r * 4 * D.d) || dalloc(&c->lowprob, r) ||
       dalloc(&c->lowprob_alt, r))
     return fail(c, BOA_E_NOMEM, "device allocation of activation buffers failed");
@@ -1283,7 +1288,8 @@ int boa_load_weights_mem(boa_ctx* c, const void* data, size_t n) {
     o.b_in = raw_at(2 * din, 2 * D.di, 1, xz_row);
     o.conv_w = raw_at(din, D.di, 4, same);
     o.conv_b = raw(din, D.di);
-    o.w_x = linear_t(D.R, din, D.di, D.ld_x, same);
+    o.w_x = linear_t(D.r + 2 * D.ds, din, D.di, D.ld_x,
+                     [&](int i) { return i < D.r ? i : i - D.r + D.rs; });
     {  // dt_proj [di][r] stored as [r][di] (no padding: read per channel)
       std::vector<float> w;
       rd.vec(w, (size_t)din * D.r);
@@ -1354,7 +1360,7 @@ int boa_load_weights_mem(boa_ctx* c, const void* data, size_t n) {
     const LayerW& L = c->layers[l];
     boa_ctx::DecW& DW = c->dlayers[l];
     dp.push_back({L.w_in, D.ld_in, 2 * D.di, D.d, 2 * D.di, 1, 0, 0, &DW.w_in});
-    dp.push_back({L.w_x, D.ld_x, D.R, D.di, c->n_xdec, 1, D.r, rb, &DW.w_x});
+    dp.push_back({L.w_x, D.ld_x, D.R, D.di, c->n_xdec, 1, D.rs, rb, &DW.w_x});
     dp.push_back({L.w_out, D.ld_out, D.d, D.di, D.d, 1, 0, 0, &DW.w_out});
     dp.push_back({L.w1, D.ld_1, 4 * D.d, D.d, 4 * D.d, 1, 0, 0, &DW.w1});
     dp.push_back({L.w2, D.ld_2, D.d, 4 * D.d, D.d, 1, 0, 0, &DW.w2});
@@ -1401,7 +1407,7 @@ int boa_load_weights_mem(boa_ctx* c, const void* data, size_t n) {
       boa_ctx::B16W &C_ = c->b16c[l], &D_ = c->b16d[l];
       bp.push_back({L.w_in, D.ld_in, 2 * D.di, D.d, 2 * D.di, 0, 0, &C_.w_in, &D_.w_in});
       bp.push_back({L.w_x, D.ld_x, D.R, D.di, D.R, 0, 0, &C_.w_x, nullptr});
-      bp.push_back({L.w_x, D.ld_x, D.R, D.di, c->n_xdec, D.r, rb, nullptr, &D_.w_x});
+      bp.push_back({L.w_x, D.ld_x, D.R, D.di, c->n_xdec, D.rs, rb, nullptr, &D_.w_x});
       bp.push_back({L.w_out, D.ld_out, D.d, D.di, D.d, 0, 0, &C_.w_out, &D_.w_out});
       bp.push_back({L.w1, D.ld_1, 4 * D.d, D.d, 4 * D.d, 0, 0, &C_.w1, &D_.w1});
       bp.push_back({L.w2, D.ld_2, D.d, 4 * D.d, D.d, 0, 0, &C_.w2, &D_.w2});
@@ -1492,10 +1498,10 @@ int boa_forward_chunk(boa_ctx* c, const uint8_t* d_tokens, int32_t lanes, int32_
 }
 
 // Rows (lanes x T) that the scratch array holds: the seven activation
-// buffers of a forward (x, xn [d]; xz [2 di]; conv, y [di]; delta [R];
+// buffers of a forward (x, xn [d]; xz [2 di]; conv, y [di]; delta [r + 2 ds];
 // hidden [4 d] floats per row), each slice aligned to 256 bytes.
 static int64_t noalloc_max_rows(const Dims& D) {
-  const int64_t per_row = 4 * (int64_t)(14 * D.d + D.R);
+  const int64_t per_row = 4 * (14 * D.d + delta_floats(D));
   return ((int64_t)kScratchBytes - 7 * 256) / per_row;
 }
 
@@ -1524,7 +1530,7 @@ int boa_forward_chunk_noalloc(boa_ctx* c, const uint8_t* d_tokens, int32_t lanes
     return p;
   };
   float *x = take(rows * D.d), *xn = take(rows * D.d), *xz = take(rows * 2 * D.di),
-        *cv = take(rows * D.di), *delta = take(rows * D.R), *y = take(rows * D.di),
+        *cv = take(rows * D.di), *delta = take(rows * delta_floats(D)), *y = take(rows * D.di),
         *hid = take(rows * 4 * D.d);
   // the context's own buffers step aside for the call; profiling (which
   // creates events) is off during it

@@ -125,9 +125,11 @@ struct LayerW {
 // (and inner channels 2 dn .. 2 d-1 of each half of in_proj's output) hold
 // zero weights, so their activations are zero, every GEMM's K-ordered chain
 // ends in exact zero terms, and the LayerNorms divide by dn.  dt_rank r is
-// dn's: ceil(dn / 16).
+// dn's: ceil(dn / 16).  A row of x_proj's output (dt inputs, B, C) has R = rs +
+// 2 ds elements, B from rs on: rs = r in fp32; in bf16 an odd r is rounded up
+// (a zero column), so that every row and its B and C start at a dword.
 struct Dims {
-  int d, L, di, r, ds, R;
+  int d, L, di, r, ds, R, rs;
   int dn;  // the model's own d_model (LayerNorm width); d = dn for the built widths
   int ld_in, ld_x, ld_out, ld_1, ld_2, ld_h1, ld_h2;
 };

@@ -575,7 +575,7 @@ struct ScanRow;
 template <int DS, int RB, bool FULL>
 struct ScanRow<DS, RB, FULL, float> {
   float d[RB], bc[2 * DS];
-  __device__ __forceinline__ ScanRow(__attribute__((address_space(4))) const float* dr, int r) {
+  __device__ __forceinline__ ScanRow(__attribute__((address_space(4))) const float* dr, int r, int) {
 #pragma unroll
     for (int j = 0; j < RB; ++j) {
       const float v = dr[j];  // j < RB <= R: inside the row
@@ -589,9 +589,9 @@ struct ScanRow<DS, RB, FULL, float> {
   __device__ __forceinline__ float C(int n) const { return bc[DS + n]; }
   __device__ __forceinline__ void between(int) const {}
 };
-// bf16 rows: dt_rank, d_state and so the row length are even (d_model is a
-// multiple of 64), so the element pairs are read as aligned dwords, widened
-// by scalar instructions where an element is used.  At d_state 32 a row's 96
+// bf16 rows: their length and B's offset rs are even (Dims), so the element
+// pairs are read as aligned dwords (scalar loads drop an address's two low
+// bits), widened by scalar instructions where an element is used.  At d_state 32 a row's 96
 // floats would not fit the SGPRs (the compiler spilled them to VGPR lanes,
 // 14 v_readlane a token): there the widening stays within groups of eight
 // states.
@@ -599,13 +599,14 @@ template <int DS, int RB, bool FULL>
 struct ScanRow<DS, RB, FULL, uint16_t> {
   uint32_t w[RB / 2], wbc[DS];
   int r;
-  __device__ __forceinline__ ScanRow(__attribute__((address_space(4))) const uint16_t* dr, int r_)
+  __device__ __forceinline__ ScanRow(__attribute__((address_space(4))) const uint16_t* dr, int r_,
+                                     int rs)
       : r(r_) {
     typedef __attribute__((address_space(4))) const uint32_t* Words;
 #pragma unroll
     for (int j = 0; j < RB / 2; ++j) w[j] = ((Words)dr)[j];
 #pragma unroll
-    for (int j = 0; j < DS; ++j) wbc[j] = ((Words)(dr + r))[j];
+    for (int j = 0; j < DS; ++j) wbc[j] = ((Words)(dr + rs))[j];
   }
   static __device__ __forceinline__ float half_of(uint32_t v, int odd) {
     return u2f(odd ? v & 0xFFFF0000u : v << 16);
@@ -674,7 +675,7 @@ void scan_chunk_sload_kernel(Dims D, LayerW Lw, const TA* __restrict__ xz,
   };
   if constexpr (M == MATH_HW) {
     auto token = [&] {
-      const ScanRow<DS, RB, FULL, TA> dv(drows, D.r);
+      const ScanRow<DS, RB, FULL, TA> dv(drows, D.r, D.rs);
       const float u = ub.load(off, at), z = zb.load(off, (int)(2u * (unsigned)at));
       yb.store(off, at, scan_token_any<DS, M>(sc.h, p, dv, scan_x<RB>(p, dv, RB), u, z));
       advance();
@@ -696,7 +697,7 @@ void scan_chunk_sload_kernel(Dims D, LayerW Lw, const TA* __restrict__ xz,
     int t = 0;
     while (t < T) {
       for (; t < T; ++t) {
-        const ScanRow<DS, RB, FULL, TA> dv(drows, D.r);
+        const ScanRow<DS, RB, FULL, TA> dv(drows, D.r, D.rs);
         const float u = ub.load(off, at), z = zb.load(off, (int)(2u * (unsigned)at));
         const float x = scan_x<RB>(p, dv, RB);
         if (!scan_ordinary(p, x, z)) break;
@@ -704,7 +705,7 @@ void scan_chunk_sload_kernel(Dims D, LayerW Lw, const TA* __restrict__ xz,
         advance();
       }
       if (t < T) {
-        const ScanRow<DS, RB, FULL, TA> dv(drows, D.r);
+        const ScanRow<DS, RB, FULL, TA> dv(drows, D.r, D.rs);
         const float u = ub.load(off, at), z = zb.load(off, (int)(2u * (unsigned)at));
         yb.store(off, at, scan_token_any<DS, M>(sc.h, p, dv, scan_x<RB>(p, dv, RB), u, z));
         advance();
@@ -776,7 +777,7 @@ __global__ __launch_bounds__(256) void scan_chunk_tblk_kernel(Dims D, LayerW Lw,
   static_assert(DS % G == 0 && TB % G == 0, "whole states and tokens per thread");
   constexpr int M = sizeof(TA) == 2 ? MATH_HW : MATH_BF;
   extern __shared__ __align__(16) float smem[];  // s_tok is read as float4
-  const int di = D.di, R = D.R, r = D.r;
+  const int di = D.di, R = D.R, r = D.r, rs = D.rs;
   const int cl = threadIdx.x % TBK_CPB, k = threadIdx.x / TBK_CPB;
   float* s_delta = smem;                                                 // [TB][R]
   float* s_tok = smem + TB * (RB + 2 * DS) + cl * S::TSTR;               // [TB][4]
@@ -850,7 +851,7 @@ __global__ __launch_bounds__(256) void scan_chunk_tblk_kernel(Dims D, LayerW Lw,
 #pragma unroll 8
     for (int tt = 0; tt < nt; ++tt) {
       const float2 dd2 = *reinterpret_cast<const float2*>(s_tok + 4 * tt);
-      const float* Bv = s_delta + tt * R + r;
+      const float* Bv = s_delta + tt * R + rs;
 #pragma unroll
       for (int n = 0; n < SPT; ++n) {
         const float dA = exp2_neg_sel<M>(na[n] * dd2.x);
@@ -869,7 +870,7 @@ __global__ __launch_bounds__(256) void scan_chunk_tblk_kernel(Dims D, LayerW Lw,
     for (int i = 0; i < TPT; ++i) {
       const int tok = k + G * i;
       if (tok < nt) {
-        const float* Cv = s_delta + tok * R + r + DS;
+        const float* Cv = s_delta + tok * R + rs + DS;
         const float* hr = s_h + tok * HS;
         float yv = 0.0f;
 #pragma unroll
@@ -949,7 +950,7 @@ hipError_t launch_scan_chunk(const Dims& D, const LayerW& Lw, const void* xz, co
                              const void* delta, float* ssm_state, void* y, int lanes, int T,
                              bool bf16, hipStream_t s) {
   const int bs = block_for(D.di);
-  if (D.r > RMAX || (D.ds != 16 && D.ds != 32)) return hipErrorInvalidValue;
+  if (D.r > RMAX || (D.ds != 16 && D.ds != 32) || (bf16 && D.rs % 2)) return hipErrorInvalidValue;
   BOA_SCAN_DISPATCH(scan_chunk_go, D, Lw, xz, conv, delta, ssm_state, y, lanes, T, bs, bf16, s);
 }
 

@@ -95,3 +95,35 @@ def test_odd_width_bf16(torch_dev, oracle, make_weights, d, ds):
     c.close()
     c2.close()
 
+
+
+@pytest.mark.parametrize("d,ds,lanes", [(72, 16, 256), (100, 16, 257), (200, 16, 128),
+                                        (200, 32, 129), (490, 16, 65), (490, 32, 64)])
+def test_odd_rank_bf16_many_lanes(torch_dev, oracle, make_weights, d, ds, lanes):
+    """An odd dt_rank (5, 7, 13, 31) at the lane counts of the scan that reads
+    the delta rows as dwords (65,536 channels in flight): the chunk forward is
+    the step's bit for bit and the oracle's within the bf16 tolerance, in odd
+    and even rows, and the container decodes to its input."""
+    torch = torch_dev
+    w = make_weights(d, 1, ds)
+    T = 5
+    rng = np.random.default_rng(d + ds)
+    tok = rng.integers(0, 256, size=(lanes, T), dtype=np.uint8)
+    want = oracle.Model(w, d, 1, ds).new_state(lanes).forward_chunk(tok)
+    c = _codec(d, 1, ds, lanes, w, "bf16")
+    c.reset_state(lanes)
+    d_log = torch.zeros(lanes * T * 256, dtype=torch.float32, device="cuda")
+    c.forward_chunk(torch.from_numpy(tok).cuda(), lanes, T, d_log)
+    torch.cuda.synchronize()
+    got = d_log.cpu().numpy().reshape(lanes, T, 256)
+    assert np.abs(got - want).max() <= 2e-2 * np.abs(want).max()
+    c.reset_state(lanes)
+    d_s = torch.zeros(lanes * 256, dtype=torch.float32, device="cuda")
+    for t in range(T):
+        c.step_batch(torch.from_numpy(np.ascontiguousarray(tok[:, t])).cuda(), lanes, d_s, True)
+        torch.cuda.synchronize()
+        assert np.array_equal(d_s.cpu().numpy().reshape(lanes, 256).view(np.uint32),
+                              got[:, t].view(np.uint32)), f"step {t}"
+    data = rng.integers(0, 256, size=lanes * 20 - 7, dtype=np.uint8).tobytes()
+    assert c.decompress(c.compress(data, chunk_size=20)) == data
+    c.close()
