@@ -60,9 +60,10 @@ constexpr float RINT_MAGIC = 12582912.0f;
 // p 2^k for k = rint_sum - RINT_MAGIC; p, p 2^k normal (or p 2^k = 2^128 = inf).
 BOA_DEV float scale_rint(float p, float rint_sum) { return u2f(f2u(p) + (f2u(rint_sum) << 23)); }
 
-// n / d, correctly rounded, for normal d with a normal reciprocal and n / d
-// zero or normal by a margin of 2^24: Newton's step on the reciprocal, then
-// two residual corrections of the quotient (Markstein).  8 instructions, 27
+// n / d, correctly rounded, for normal d with a normal reciprocal, n / d zero
+// or normal, and n zero or |n| >= 2^-100 (so that the residuals n - d q do not
+// underflow): Newton's step on the reciprocal, then two residual corrections
+// of the quotient (Markstein).  8 instructions, 27
 // cycles, against 12 and about 45 for the scaled division.
 BOA_DEV float div_normal(float n, float d) {
   float y = __builtin_amdgcn_rcpf(d);
