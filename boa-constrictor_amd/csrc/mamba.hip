@@ -661,9 +661,8 @@ void scan_chunk_sload_kernel(Dims D, LayerW Lw, const TA* __restrict__ xz,
   CIn drows = (CIn)(delta + (size_t)b * T * R);
   // u, z and y through buffer accesses: a lane's byte offset in the row is
   // constant and the row's offset a scalar, so a token costs no vector
-  // address arithmetic.  A lane's rows span under 2^32 bytes: with 65,536
-  // channels in flight (the dispatch's lower bound) their activations would
-  // otherwise exceed the card's memory 100 times.
+  // address arithmetic.  The dispatch takes lanes whose rows span less than
+  // 2^32 bytes.
   const RowBuf<TA> ub(conv + (size_t)b * T * di), zb(xz + ((size_t)b * T * 2 + 1) * di),
       yb(y + (size_t)b * T * di);
   const int off = (int)(c * sizeof(TA)), row = di * (int)sizeof(TA);
@@ -902,7 +901,11 @@ static hipError_t scan_chunk_go(const Dims& D, const LayerW& Lw, const void* xz,
                                 const void* delta, float* ssm_state, void* y, int lanes, int T,
                                 int bs, bool bf16, hipStream_t s) {
   const dim3 grid(lanes * ((D.di + bs - 1) / bs));
-  if ((int64_t)lanes * D.di < BOA_SCAN_TBLK_BELOW) {
+  // Rows of a lane that span 2^32 bytes are beyond the other form's 32-bit
+  // offsets (with 65,536 channels in flight a forward's activations would then
+  // take 0.9 TB or more: 64 lanes of 524,288 tokens, d_model 512).
+  const int64_t span = (int64_t)T * 2 * D.di * (bf16 ? 2 : 4);
+  if ((int64_t)lanes * D.di < BOA_SCAN_TBLK_BELOW || span >= (1ll << 32)) {
     if (D.di % TBK_CPB) return hipErrorInvalidValue;
     const size_t lds = sizeof(float) * TblkShape<DS>::template lds_floats<RB>();
     const dim3 g2((lanes * D.di) / TBK_CPB);
