@@ -195,7 +195,7 @@ __device__ __forceinline__ float scan_x_max(const float (&na)[DS]) {
     lo = __builtin_fminf(lo, na[n]);
     nan = nan || na[n] != na[n];
   }
-  const float x = 126.0f / -lo - 0.7f;  // lo = 0: inf
+  const float x = 126.0f / __builtin_fabsf(lo) - 0.7f;  // lo = -0 or 0: inf
   return !nan && x >= 0.0f ? __builtin_fminf(x, ORDINARY) : -__builtin_huge_valf();
 }
 

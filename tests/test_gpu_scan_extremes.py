@@ -91,3 +91,27 @@ def test_decode_limits_match_the_oracle(oracle, tmp_path, d, lanes):
     assert blob == oracle.Model(w, d, 1).compress(tok.tobytes(), chunk_size=T)
     assert c.decompress(blob) == tok.tobytes()
     c.close()
+
+
+def test_no_decay_matches_the_oracle(oracle, tmp_path):
+    """A_log below -87: every decay coefficient is -0, the exponents are -0 and
+    every ordinary token's scan runs without clamps."""
+    import torch
+
+    import boa_hip
+    d, T = 64, 9
+    w = tmp_path / "w.bin"
+    synth.write_weights(str(w), [(name, np.full_like(a, -90.0) if name.endswith("A_log") else a)
+                                 for name, a in synth.random_weight_tensors(d, 1, 16, seed=5)])
+    lanes = 64 * 1024 // (2 * d)
+    tok = np.random.default_rng(d).integers(0, 256, size=(lanes, T), dtype=np.uint8)
+    want = oracle.Model(w, d, 1, 16).new_state(lanes).forward_chunk(tok)
+    c = boa_hip.Codec(d, 1, 16, lanes)
+    c.set_stream(torch.cuda.current_stream().cuda_stream)
+    c.load_weights(w)
+    c.reset_state(lanes)
+    got = torch.zeros((lanes, T, 256), device="cuda")
+    c.forward_chunk(torch.from_numpy(tok).cuda(), lanes, T, got)
+    torch.cuda.synchronize()
+    assert np.array_equal(got.cpu().numpy().view(np.uint32), want.view(np.uint32))
+    c.close()
