@@ -551,11 +551,13 @@ __global__ __launch_bounds__(512, 2) void gemm_bf16_persist_kernel(GemmB16Args a
 
 // What the kernel's addressing takes: whole 256-feature tiles up to
 // GP_MAX_N, whole 64-k stages, 16-byte rows, a tile's rows within 32-bit byte
-// offsets; a residual or a bf16 copy only beside fp32 output.
+// offsets; a residual or a bf16 copy only beside fp32 output, an activation
+// only beside bf16 output (the model has no others).
 static bool b16_persist_fits(const GemmB16Args& a) {
   return a.N % 256 == 0 && a.N <= GP_MAX_N && a.K % 64 == 0 && a.K >= 64 && a.ldx % 8 == 0 &&
          a.ldw % 8 == 0 && a.ldw >= a.K && a.ldx <= (1 << 20) && a.ldw <= (1 << 20) &&
-         a.ldc % 8 == 0 && (!a.res || a.ldr % 4 == 0) && (!a.c_bf16 || (!a.res && !a.C2));
+         a.ldc % 8 == 0 && (!a.res || a.ldr % 4 == 0) &&
+         (a.c_bf16 ? !a.res && !a.C2 : a.act == ACT_NONE);
 }
 
 static hipError_t launch_b16_persist(const GemmB16Args& a, hipStream_t s) {
@@ -563,16 +565,16 @@ static hipError_t launch_b16_persist(const GemmB16Args& a, hipStream_t s) {
   // a multiple of eight blocks (one share of the XCDs each), at most one per CU
   const long long tiles = (long long)((m_blocks + 7) / 8) * (a.N / 256) * 8;
   const unsigned grid = (unsigned)std::min<long long>(tiles, 256);
-#define BOA_B16_GO(ACTv)                                                                       \
-  if (a.c_bf16)                                                                                \
-    BOA_LAUNCH((gemm_bf16_persist_kernel<ACTv, false>), dim3(grid), dim3(512), 0, s, a,        \
-               m_blocks);                                                                      \
-  else                                                                                         \
-    BOA_LAUNCH((gemm_bf16_persist_kernel<ACTv, true>), dim3(grid), dim3(512), 0, s, a, m_blocks)
+#define BOA_B16_GO(ACTv, F32v)                                                                  \
+  BOA_LAUNCH((gemm_bf16_persist_kernel<ACTv, F32v>), dim3(grid), dim3(512), 0, s, a, m_blocks)
+  if (!a.c_bf16) {
+    BOA_B16_GO(ACT_NONE, true);
+    return hipGetLastError();
+  }
   switch (a.act) {
-    case ACT_NONE: BOA_B16_GO(ACT_NONE); break;
-    case ACT_GELU: BOA_B16_GO(ACT_GELU); break;
-    case ACT_RELU: BOA_B16_GO(ACT_RELU); break;
+    case ACT_NONE: BOA_B16_GO(ACT_NONE, false); break;
+    case ACT_GELU: BOA_B16_GO(ACT_GELU, false); break;
+    case ACT_RELU: BOA_B16_GO(ACT_RELU, false); break;
     default: return hipErrorInvalidValue;
   }
 #undef BOA_B16_GO
@@ -929,6 +931,7 @@ constexpr int FR_LDS = FR_ST + 1024;
 
 template <int LNF>
 __global__ __launch_bounds__(256, 2) void ffn_bf16_rows_kernel(FfnB16Args a) {
+  static_assert((LNF & 1) != 0, "LN2 is always applied here");
   constexpr int D = 256, H = 1024;
   __shared__ __attribute__((aligned(16))) unsigned char fr_smem[FR_LDS];
   const int tid = threadIdx.x, lane = tid & 63;
@@ -956,7 +959,7 @@ __global__ __launch_bounds__(256, 2) void ffn_bf16_rows_kernel(FfnB16Args a) {
   b2s[tid] = a.b2 ? a.b2[tid] : 0.0f;
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   __syncthreads();
-  if constexpr ((LNF & 1) != 0) {  // one thread per row, elements in order
+  {  // one thread per row, elements in order
     if (tid < 128) {
       const unsigned char* row = fr_smem + tid * 128;
       float sm = 0.0f, sq = 0.0f;
@@ -1011,7 +1014,7 @@ __global__ __launch_bounds__(256, 2) void ffn_bf16_rows_kernel(FfnB16Args a) {
           ch * 64 + i * (16 * H * 2), 0, 0);
   };
   copy(0, 0);
-  if constexpr ((LNF & 1) != 0) {  // LN2 in the registers while the first stage lands
+  {  // LN2 in the registers while the first stage lands
 #pragma unroll
     for (int p = 0; p < 2; ++p) {
       const int row = 32 * wave + 16 * p + j;
@@ -1232,7 +1235,7 @@ __global__ __launch_bounds__(256, 2) void ffn_bf16_rows_kernel(FfnB16Args a) {
 // More blocks than CUs: by rows.  Up to one block per CU the 16 waves hide
 // more of a block's own latencies (a forward call, two layers: 32,768 rows 1809
 // us against 1824, 1000 rows 259 against 271; 33,000 rows 1950 against 1888,
-// 65,535 rows 3519 against 3449).
+// 65,535 rows 3519 against 3449).  By rows only with LN2 in the kernel.
 hipError_t ffn_bf16(const FfnB16Args& args, hipStream_t s) {
   FfnB16Args a = args;
   if (a.n <= 0) a.n = a.D;  // the LayerNorms' width defaults to the row width
@@ -1243,20 +1246,18 @@ hipError_t ffn_bf16(const FfnB16Args& args, hipStream_t s) {
       const bool ln2 = a.ln2_w && a.ln2_b, ln1 = a.xn && a.ln1_w && a.ln1_b;
       if ((a.ln2_w || a.ln2_b) && !ln2) return hipErrorInvalidValue;
       if ((a.xn || a.ln1_w || a.ln1_b) && !ln1) return hipErrorInvalidValue;
-#define BOA_FFN(F)                                                                      \
-  if (blocks > 256)                                                                     \
-    BOA_LAUNCH((ffn_bf16_rows_kernel<F>), dim3(blocks), dim3(256), 0, s, a);            \
-  else                                                                                  \
-    BOA_LAUNCH((ffn_bf16_kernel<256, 128, 64, 4, 4, 4, 4, F>), dim3(blocks), dim3(1024), 0, s, a)
-      if (ln2 && ln1) {
-        BOA_FFN(3);
-      } else if (ln2) {
-        BOA_FFN(1);
-      } else if (ln1) {
-        BOA_FFN(2);
-      } else {
-        BOA_FFN(0);
-      }
+      const bool rows = blocks > 256 && ln2;
+#define BOA_FFN(F)                                                                            \
+  BOA_LAUNCH((ffn_bf16_kernel<256, 128, 64, 4, 4, 4, 4, F>), dim3(blocks), dim3(1024), 0, s, a)
+#define BOA_FFN_ROWS(F) \
+  BOA_LAUNCH((ffn_bf16_rows_kernel<F>), dim3(blocks), dim3(256), 0, s, a)
+      if (rows && ln1) BOA_FFN_ROWS(3);
+      else if (rows) BOA_FFN_ROWS(1);
+      else if (ln2 && ln1) BOA_FFN(3);
+      else if (ln2) BOA_FFN(1);
+      else if (ln1) BOA_FFN(2);
+      else BOA_FFN(0);
+#undef BOA_FFN_ROWS
 #undef BOA_FFN
       break;
     }
