@@ -164,15 +164,16 @@ __device__ __forceinline__ void pd_ln_apply(const float* xs, float* xn, const fl
 // phases (the scan's 16 exponentials per channel, GELU, the CDF) scale with
 // LP.  Fewer lanes per block spread those phases over more CUs.
 //
-// What bounds it: a serial chain.  A step is 30 phases between barriers, in
-// which an MFMA chain of K / 4 takes 42 cycles per MFMA (256 features at once:
-// 2048 cycles a SIMD), and the elementwise phases their instruction latency.
+// What bounds it: a serial chain.  A step is 10 L + 4 phases between barriers
+// (24 at two layers), in which an MFMA chain of K / 4 takes 42 cycles per MFMA
+// (256 features at once: 2048 cycles a SIMD), and the elementwise phases their
+// instruction latency.
 // So everything that does not depend on the phase before is out of the chain:
 // weights and recurrent states are loaded phases ahead into registers, MFMA
 // outputs of LP < 16 lanes are spread over the wave before GELU and the conv
 // step, the coder's division runs under out_proj, and the symbol search stays
 // in the registers of the CDF (µs per step at 2 layers: 1 to 512 lanes 34.7 ->
-// 25.5, 1024 lanes 42.8 -> 27.9, 4096 lanes 58.7 -> 40.4; 2 lanes per block
+// 25.5, 1024 lanes 42.8 -> 27.8, 4096 lanes 58.7 -> 39.9; 2 lanes per block
 // gave 25.0 up to 300 lanes, 26.5 at 512).
 template <int NB, int RB, int LP>
 __global__ __launch_bounds__(1024) void dec_persist_kernel(PersistArgs a) {

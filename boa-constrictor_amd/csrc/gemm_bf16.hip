@@ -583,10 +583,10 @@ static hipError_t launch_b16_persist(const GemmB16Args& a, hipStream_t s) {
 
 // W must hold round_up(N, 256) rows (zero padded) for every configuration.
 // Outputs of whole 256-feature tiles run on the persistent blocks (TFLOP/s at
-// M about 10^6, against the 256 x 256 blocks of gemm_bf16_kernel: K 256 N
-// 1024 435 -> 694, K 512 N 256 594 -> 819, K 512 N 2048 667 -> 946, K 1024 N
-// 512 799 -> 1064, K 2048 N 512 with residual 657 -> 855, GELU K 512 N 2048
-// 540 -> 731; M 255 to 1300 as fast or faster); narrower or unaligned ones
+// M = 2^20, against the 16-wave 256 x 256 blocks of gemm_bf16_kernel: K 256 N
+// 1024 492 -> 766, K 512 N 256 625 -> 842, K 512 N 2048 688 -> 1007, K 1024 N
+// 512 839 -> 1066, K 2048 N 512 with residual 822 -> 982, GELU K 512 N 2048
+// 590 -> 781; M 255 to 1300 as fast or faster); narrower or unaligned ones
 // (x_proj, d_model 64's and 128's narrow outputs) on 128 x 64 blocks with 8
 // waves.
 hipError_t gemm_bf16(const GemmB16Args& a, hipStream_t s) {
