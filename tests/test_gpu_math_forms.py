@@ -4,6 +4,7 @@ ordinary arguments and in waves that mix them with special ones; and the plain
 forms are the CPU oracle's."""
 import ctypes
 import os
+import subprocess
 
 import numpy as np
 import pytest
@@ -16,7 +17,11 @@ FORMS = ["expf_", "expf_br", "exp2_neg", "sigmoid", "sigmoid_br", "softplus", "s
 
 @pytest.fixture(scope="module")
 def lib():
-    return ctypes.CDLL(os.path.join(os.path.dirname(os.path.abspath(__file__)), "libmath_forms.so"))
+    here = os.path.dirname(os.path.abspath(__file__))
+    so = os.path.join(here, "libmath_forms.so")
+    if not os.path.exists(so):
+        subprocess.run(["make", "-s", "-C", here], check=True)
+    return ctypes.CDLL(so)
 
 
 @pytest.mark.parametrize("scatter", [0, 1])
