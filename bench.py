@@ -610,7 +610,7 @@ def main() -> int:
                "isa": {"v4": "x86-64-v4 (AVX-512)", "v3": "x86-64-v3 (AVX2 + FMA)"}.get(cb["isa"], cb["isa"]),
                "build": f"gcc -O3 -march=x86-64-{cb['isa']} -ffp-contract=off -fopenmp ({cb['lib']})",
                "host": info,
-               "threads_rule": "OMP_NUM_THREADS of the GPU box (its CPU share for one GPU), "
+               "threads_rule": "OMP_NUM_THREADS where it is set (the CPU share of one GPU), "
                                "else every core in the process's affinity mask"}
 
     out = {
