@@ -553,6 +553,13 @@ hipError_t launch_conv_chunk(const void* xz, float* conv_state, const float* w, 
 }
 
 // -------------------------------------------------------- selective scan
+// The element at which a row's B starts (in fp32 rs = r: no further kernel
+// argument, which the token-blocked form's loop showed, 0.7 %).
+template <typename TA>
+__device__ __forceinline__ int row_b(const Dims& D) {
+  return sizeof(TA) == 2 ? D.rs : D.r;
+}
+
 // Thread per (lane, channel); a block covers bs channels of one lane, so the
 // token's delta row (dt_in | B | C) is the same for every thread of the wave
 // and is read with scalar loads into SGPRs: no LDS staging and no barriers
@@ -575,7 +582,8 @@ struct ScanRow;
 template <int DS, int RB, bool FULL>
 struct ScanRow<DS, RB, FULL, float> {
   float d[RB], bc[2 * DS];
-  __device__ __forceinline__ ScanRow(__attribute__((address_space(4))) const float* dr, int r, int) {
+  __device__ __forceinline__ ScanRow(__attribute__((address_space(4))) const float* dr, const Dims& D) {
+    const int r = D.r;
 #pragma unroll
     for (int j = 0; j < RB; ++j) {
       const float v = dr[j];  // j < RB <= R: inside the row
@@ -591,22 +599,22 @@ struct ScanRow<DS, RB, FULL, float> {
 };
 // bf16 rows: their length and B's offset rs are even (Dims), so the element
 // pairs are read as aligned dwords (scalar loads drop an address's two low
-// bits), widened by scalar instructions where an element is used.  At d_state 32 a row's 96
-// floats would not fit the SGPRs (the compiler spilled them to VGPR lanes,
-// 14 v_readlane a token): there the widening stays within groups of eight
-// states.
+// bits), widened by scalar instructions where an element is used.  At d_state
+// 32 a row's 96 floats would not fit the SGPRs (the compiler spilled them to
+// VGPR lanes, 14 v_readlane a token): there the widening stays within groups
+// of eight states.
 template <int DS, int RB, bool FULL>
 struct ScanRow<DS, RB, FULL, uint16_t> {
   uint32_t w[RB / 2], wbc[DS];
   int r;
-  __device__ __forceinline__ ScanRow(__attribute__((address_space(4))) const uint16_t* dr, int r_,
-                                     int rs)
-      : r(r_) {
+  __device__ __forceinline__ ScanRow(__attribute__((address_space(4))) const uint16_t* dr,
+                                     const Dims& D)
+      : r(D.r) {
     typedef __attribute__((address_space(4))) const uint32_t* Words;
 #pragma unroll
     for (int j = 0; j < RB / 2; ++j) w[j] = ((Words)dr)[j];
 #pragma unroll
-    for (int j = 0; j < DS; ++j) wbc[j] = ((Words)(dr + rs))[j];
+    for (int j = 0; j < DS; ++j) wbc[j] = ((Words)(dr + row_b<uint16_t>(D)))[j];
   }
   static __device__ __forceinline__ float half_of(uint32_t v, int odd) {
     return u2f(odd ? v & 0xFFFF0000u : v << 16);
@@ -674,7 +682,7 @@ void scan_chunk_sload_kernel(Dims D, LayerW Lw, const TA* __restrict__ xz,
   };
   if constexpr (M == MATH_HW) {
     auto token = [&] {
-      const ScanRow<DS, RB, FULL, TA> dv(drows, D.r, D.rs);
+      const ScanRow<DS, RB, FULL, TA> dv(drows, D);
       const float u = ub.load(off, at), z = zb.load(off, (int)(2u * (unsigned)at));
       yb.store(off, at, scan_token_any<DS, M>(sc.h, p, dv, scan_x<RB>(p, dv, RB), u, z));
       advance();
@@ -696,7 +704,7 @@ void scan_chunk_sload_kernel(Dims D, LayerW Lw, const TA* __restrict__ xz,
     int t = 0;
     while (t < T) {
       for (; t < T; ++t) {
-        const ScanRow<DS, RB, FULL, TA> dv(drows, D.r, D.rs);
+        const ScanRow<DS, RB, FULL, TA> dv(drows, D);
         const float u = ub.load(off, at), z = zb.load(off, (int)(2u * (unsigned)at));
         const float x = scan_x<RB>(p, dv, RB);
         if (!scan_ordinary(p, x, z)) break;
@@ -704,7 +712,7 @@ void scan_chunk_sload_kernel(Dims D, LayerW Lw, const TA* __restrict__ xz,
         advance();
       }
       if (t < T) {
-        const ScanRow<DS, RB, FULL, TA> dv(drows, D.r, D.rs);
+        const ScanRow<DS, RB, FULL, TA> dv(drows, D);
         const float u = ub.load(off, at), z = zb.load(off, (int)(2u * (unsigned)at));
         yb.store(off, at, scan_token_any<DS, M>(sc.h, p, dv, scan_x<RB>(p, dv, RB), u, z));
         advance();
@@ -776,7 +784,7 @@ __global__ __launch_bounds__(256) void scan_chunk_tblk_kernel(Dims D, LayerW Lw,
   static_assert(DS % G == 0 && TB % G == 0, "whole states and tokens per thread");
   constexpr int M = sizeof(TA) == 2 ? MATH_HW : MATH_BF;
   extern __shared__ __align__(16) float smem[];  // s_tok is read as float4
-  const int di = D.di, R = D.R, r = D.r, rs = D.rs;
+  const int di = D.di, R = D.R, r = D.r, rs = row_b<TA>(D);
   const int cl = threadIdx.x % TBK_CPB, k = threadIdx.x / TBK_CPB;
   float* s_delta = smem;                                                 // [TB][R]
   float* s_tok = smem + TB * (RB + 2 * DS) + cl * S::TSTR;               // [TB][4]
@@ -953,7 +961,8 @@ hipError_t launch_scan_chunk(const Dims& D, const LayerW& Lw, const void* xz, co
                              const void* delta, float* ssm_state, void* y, int lanes, int T,
                              bool bf16, hipStream_t s) {
   const int bs = block_for(D.di);
-  if (D.r > RMAX || (D.ds != 16 && D.ds != 32) || (bf16 && D.rs % 2)) return hipErrorInvalidValue;
+  if (D.r > RMAX || (D.ds != 16 && D.ds != 32) || (bf16 ? D.rs % 2 : D.rs != D.r))
+    return hipErrorInvalidValue;
   BOA_SCAN_DISPATCH(scan_chunk_go, D, Lw, xz, conv, delta, ssm_state, y, lanes, T, bs, bf16, s);
 }
 
