@@ -580,8 +580,10 @@ static hipError_t launch_cfg(const GemmArgs& a, hipStream_t s, int swizzle = 1) 
 // wait for fewer operands: 128x64 blocks hold eight times the work and are 10
 // to 17 % cheaper for it from K 256 on, so they have to come to less than 1/7 of
 // the number; 64x32 blocks of eight waves twice, 2 to 5 % cheaper from K 512
-// on (below they gain and lose 4 %), so they have to come to half of it.  One
-// of either on a CU exposes its latency (N 256 K 512, 3000 rows: 27.7 us of
+// on, so they have to come to half of it; at K 256 that holds for whole rounds
+// of the four that a CU holds (N 256, 8064 rows, 4 on the fullest: 16.4 us
+// against 17.7; 10,180 rows, 5: 21.1 against 20.6), below nowhere.  One of
+// either on a CU exposes its latency (N 256 K 512, 3000 rows: 27.7 us of
 // 128x64, 14.1 of 32x32).  us of 128x64 / 64x32 / 32x32 (blocks on the fullest
 // CU): N 1024 K 256 at 8064 rows 46.7 / 50.5 / 50.8 (4, 16, 32), at 6387 46.1 /
 // 42.0 / 41.6 (4, 13, 25), at 1178 16.4 / 12.8 / 11.4 (2, 3, 5); N 256 K 1024
@@ -594,7 +596,9 @@ int gemm_f32_config(const GemmArgs& a) {
   const long long n128 = cu_blocks(a, 128, 64), n64 = cu_blocks(a, 64, 32),
                   n32 = cu_blocks(a, 32, 32);
   if (a.K >= 256 && n128 >= 2 && 7 * n128 < n32) return 1;
-  if (a.K >= 512 && a.K % 32 == 0 && n64 >= 2 && 2 * n64 == n32) return 3;
+  if (a.K % 32 == 0 && 2 * n64 == n32 &&
+      (a.K >= 512 ? n64 >= 2 : a.K >= 256 && n64 % 4 == 0))
+    return 3;
   return 2;
 }
 
