@@ -9,21 +9,20 @@ namespace boa {
 
 // value = bias + x[t-3] w0 + x[t-2] w1 + x[t-1] w2 + x[t] w3 (unfused, k
 // order), then SiLU.  The state holds the last four inputs, most recent last.
-template <int M = MATH_BF>
-__device__ __forceinline__ float conv_value(float bias, float xm3, float xm2, float xm1, float x0,
-                                            const float4 w) {
+__device__ __forceinline__ float conv_sum(float bias, float xm3, float xm2, float xm1, float x0,
+                                          const float4 w) {
   float v = bias;
   v = v + xm3 * w.x;
   v = v + xm2 * w.y;
   v = v + xm1 * w.z;
   v = v + x0 * w.w;
-  return silu<M>(v);
+  return v;
 }
 
 // Step form: state s = (x[t-4], x[t-3], x[t-2], x[t-1]), new input x0.
 template <int M = MATH_BF>
 __device__ __forceinline__ float conv_step_value(float bias, float4 s, float x0, const float4 w) {
-  return conv_value<M>(bias, s.y, s.z, s.w, x0, w);
+  return silu<M>(conv_sum(bias, s.y, s.z, s.w, x0, w));
 }
 
 // Decode-step activation layouts, lane capacity ld:

@@ -246,6 +246,27 @@ BOA_DEV float sigmoid(float x) {
 template <int M = MATH_BF>
 BOA_DEV float silu(float x) { return x * sigmoid<M>(x); }
 
+// ... of N values at once, one form for all of them: one branch, their chains
+// side by side
+template <int M, int N>
+BOA_DEV void silu_each(float (&v)[N]) {
+  if constexpr (M == MATH_HW) {
+#pragma unroll
+    for (int k = 0; k < N; ++k) v[k] = silu<M>(v[k]);
+  } else {
+    bool ordinary = true;
+#pragma unroll
+    for (int k = 0; k < N; ++k) ordinary &= __builtin_fabsf(v[k]) <= ORDINARY;
+    if (wave_ordinary(ordinary)) {
+#pragma unroll
+      for (int k = 0; k < N; ++k) v[k] = v[k] * sigmoid_core(v[k]);
+    } else {
+#pragma unroll
+      for (int k = 0; k < N; ++k) v[k] = v[k] * sigmoid_any<M>(v[k]);
+    }
+  }
+}
+
 // unthresholded softplus log(1 + exp(x)) (inference_kernels.cu:376-382)
 template <int M = MATH_BF>
 BOA_DEV float softplus(float x) {

@@ -437,7 +437,13 @@ __global__ __launch_bounds__(256) void conv_chunk_tp_kernel(const TA* __restrict
                                                             TA* __restrict__ out, int lanes, int T,
                                                             int di, int ntb) {
   constexpr int SB = 8;  // tokens loaded together
-  static_assert(TB % SB == 0, "whole sub-blocks");
+  // Tokens whose SiLUs share a branch: one value at a time, the chains run one
+  // after the other and a small grid shows their latency (290 rows, d_model
+  // 256: 8.5 us; one token 7.5, two 7.2, eight 7.0; branch-free 7.8); eight
+  // take the registers that a large one needs (10^6 rows: 951, 952, 947, 1043
+  // us; branch-free 983).
+  constexpr int G = 2;
+  static_assert(TB % SB == 0 && SB % G == 0, "whole sub-blocks");
   const int dq = di / CP;
   const int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (idx >= (int64_t)lanes * ntb * dq) return;
@@ -478,14 +484,19 @@ __global__ __launch_bounds__(256) void conv_chunk_tp_kernel(const TA* __restrict
 #pragma unroll
     for (int v = 0; v < SB; ++v) ldcp<CP>(xp + (size_t)(t0 + u + v) * 2 * di, xv[v]);
 #pragma unroll
-    for (int v = 0; v < SB; ++v) {
-      float o[CP];
+    for (int v = 0; v < SB; v += G) {
+      float o[G * CP];
 #pragma unroll
-      for (int k = 0; k < CP; ++k) {
-        o[k] = conv_value<M>(bias[k], xm3[k], xm2[k], xm1[k], xv[v][k], wv[k]);
-        xm3[k] = xm2[k]; xm2[k] = xm1[k]; xm1[k] = xv[v][k];
-      }
-      stcp<CP>(op + (size_t)(t0 + u + v) * di, o);
+      for (int i = 0; i < G; ++i)
+#pragma unroll
+        for (int k = 0; k < CP; ++k) {
+          const float x0 = xv[v + i][k];
+          o[i * CP + k] = conv_sum(bias[k], xm3[k], xm2[k], xm1[k], x0, wv[k]);
+          xm3[k] = xm2[k]; xm2[k] = xm1[k]; xm1[k] = x0;
+        }
+      silu_each<M>(o);
+#pragma unroll
+      for (int i = 0; i < G; ++i) stcp<CP>(op + (size_t)(t0 + u + v + i) * di, o + i * CP);
     }
   }
   for (; u < nt; ++u) {  // the tile's last tokens
@@ -493,9 +504,10 @@ __global__ __launch_bounds__(256) void conv_chunk_tp_kernel(const TA* __restrict
     ldcp<CP>(xp + (size_t)(t0 + u) * 2 * di, x0);
 #pragma unroll
     for (int k = 0; k < CP; ++k) {
-      o[k] = conv_value<M>(bias[k], xm3[k], xm2[k], xm1[k], x0[k], wv[k]);
+      o[k] = conv_sum(bias[k], xm3[k], xm2[k], xm1[k], x0[k], wv[k]);
       xm3[k] = xm2[k]; xm2[k] = xm1[k]; xm1[k] = x0[k];
     }
+    silu_each<M>(o);
     stcp<CP>(op + (size_t)(t0 + u) * di, o);
   }
   if (tb == 0) {
