@@ -457,7 +457,9 @@ __global__ __launch_bounds__(512, 2) void gemm_bf16_persist_kernel(GemmB16Args a
       else if (ACT == ACT_RELU) t = fmaxf(0.0f, t);
       return t;
     };
-    if constexpr (!F32) {
+    if (!full && m0 >= a.M) {  // padding rows only: no activations, no stores
+      pending = 0;
+    } else if constexpr (!F32) {
 #pragma unroll
       for (int half = 0; half < 2; ++half) {  // features 64 half .. of the wave's 128
         lds_u32x4 bv[4];
