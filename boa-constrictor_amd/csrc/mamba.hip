@@ -437,12 +437,13 @@ __global__ __launch_bounds__(256) void conv_chunk_tp_kernel(const TA* __restrict
                                                             TA* __restrict__ out, int lanes, int T,
                                                             int di, int ntb) {
   constexpr int SB = 8;  // tokens loaded together
-  // Tokens whose SiLUs share a branch: one value at a time, the chains run one
-  // after the other and a small grid shows their latency (290 rows, d_model
-  // 256: 8.5 us; one token 7.5, two 7.2, eight 7.0; branch-free 7.8); eight
-  // take the registers that a large one needs (10^6 rows: 951, 952, 947, 1043
-  // us; branch-free 983).
-  constexpr int G = 2;
+  constexpr int M = sizeof(TA) == 2 ? MATH_HW : MATH_BF;
+  // Tokens whose SiLUs share a branch (bf16's have none): one value at a time,
+  // the chains run one after the other and a small grid shows their latency
+  // (290 rows, d_model 256: 8.5 us; one token 7.5, two 7.2, eight 7.0;
+  // branch-free 7.8); eight take the registers that a large one needs (10^6
+  // rows: 951, 952, 947, 1043 us; branch-free 983).
+  constexpr int G = M == MATH_HW ? 1 : 2;
   static_assert(TB % SB == 0 && SB % G == 0, "whole sub-blocks");
   const int dq = di / CP;
   const int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -451,7 +452,6 @@ __global__ __launch_bounds__(256) void conv_chunk_tp_kernel(const TA* __restrict
   const int64_t rest = idx / dq;
   const int tb = (int)(rest % ntb), b = (int)(rest / ntb);
   const int t0 = tb * TB;
-  constexpr int M = sizeof(TA) == 2 ? MATH_HW : MATH_BF;
   float4 wv[CP];
   float bias[CP];
 #pragma unroll
