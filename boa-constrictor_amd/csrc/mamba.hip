@@ -565,13 +565,6 @@ hipError_t launch_conv_chunk(const void* xz, float* conv_state, const float* w, 
 }
 
 // -------------------------------------------------------- selective scan
-// The element at which a row's B starts (in fp32 rs = r: no further kernel
-// argument, which the token-blocked form's loop showed, 0.7 %).
-template <typename TA>
-__device__ __forceinline__ int row_b(const Dims& D) {
-  return sizeof(TA) == 2 ? D.rs : D.r;
-}
-
 // Thread per (lane, channel); a block covers bs channels of one lane, so the
 // token's delta row (dt_in | B | C) is the same for every thread of the wave
 // and is read with scalar loads into SGPRs: no LDS staging and no barriers
@@ -626,7 +619,7 @@ struct ScanRow<DS, RB, FULL, uint16_t> {
 #pragma unroll
     for (int j = 0; j < RB / 2; ++j) w[j] = ((Words)dr)[j];
 #pragma unroll
-    for (int j = 0; j < DS; ++j) wbc[j] = ((Words)(dr + row_b<uint16_t>(D)))[j];
+    for (int j = 0; j < DS; ++j) wbc[j] = ((Words)(dr + D.rs))[j];
   }
   static __device__ __forceinline__ float half_of(uint32_t v, int odd) {
     return u2f(odd ? v & 0xFFFF0000u : v << 16);
@@ -796,7 +789,8 @@ __global__ __launch_bounds__(256) void scan_chunk_tblk_kernel(Dims D, LayerW Lw,
   static_assert(DS % G == 0 && TB % G == 0, "whole states and tokens per thread");
   constexpr int M = sizeof(TA) == 2 ? MATH_HW : MATH_BF;
   extern __shared__ __align__(16) float smem[];  // s_tok is read as float4
-  const int di = D.di, R = D.R, r = D.r, rs = row_b<TA>(D);
+  // rs (Dims) from r: as one more kernel argument it slowed the loop by 0.7 %
+  const int di = D.di, R = D.R, r = D.r, rs = sizeof(TA) == 2 ? (r + 1) & ~1 : r;
   const int cl = threadIdx.x % TBK_CPB, k = threadIdx.x / TBK_CPB;
   float* s_delta = smem;                                                 // [TB][R]
   float* s_tok = smem + TB * (RB + 2 * DS) + cl * S::TSTR;               // [TB][4]
@@ -973,7 +967,7 @@ hipError_t launch_scan_chunk(const Dims& D, const LayerW& Lw, const void* xz, co
                              const void* delta, float* ssm_state, void* y, int lanes, int T,
                              bool bf16, hipStream_t s) {
   const int bs = block_for(D.di);
-  if (D.r > RMAX || (D.ds != 16 && D.ds != 32) || (bf16 ? D.rs % 2 : D.rs != D.r))
+  if (D.r > RMAX || (D.ds != 16 && D.ds != 32) || D.rs != (bf16 ? (D.r + 1) & ~1 : D.r))
     return hipErrorInvalidValue;
   BOA_SCAN_DISPATCH(scan_chunk_go, D, Lw, xz, conv, delta, ssm_state, y, lanes, T, bs, bf16, s);
 }
